@@ -128,6 +128,20 @@ DEV float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 DEV float fast_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 DEV float fast_rsq(float x) { return __builtin_amdgcn_rsqf(x); }
 
+// max(x, lo) and min(x, hi) with a wave-uniform bound, as one instruction (the
+// library forms first canonicalize both operands).  A NaN x gives the bound,
+// as fmaxf and fminf do.
+DEV float max_s(float x, float lo) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "s"(lo), "v"(x));
+    return r;
+}
+DEV float min_s(float x, float hi) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "s"(hi), "v"(x));
+    return r;
+}
+
 // LDS atomic subtract without a returned value (ds_sub_u32; HIP's atomicSub
 // would negate and add).
 DEV void lds_sub(int* p, int v) {
@@ -220,12 +234,17 @@ DEV float4 load_pt<ADGPU_MAP_BF16>(const void* base, uint32_t idx) {
 // LDS layout
 // ---------------------------------------------------------------------------
 struct SharedView {           // staged once per workgroup
-    const PairA* pa;          // LDS (or global when the pairs do not fit)
-    const PairB* pb;
+    const PairA* pa;          // LDS (or global when the pairs do not fit): record p of step k is
+    const PairB* pb;          //   [k * pair_stride<TW, PL> + lane] of both
+    const uint32_t* px;       // flags, global (read for exponents other than 12-6 / 12-10)
     const float4* tor_unit;
     const float4* tor_move;
     const int2* tor_atoms;
 };
+
+// Element at byte offset `bytes` of an array.
+template <class V>
+DEV V* at(V* p, uint32_t bytes) { return reinterpret_cast<V*>(reinterpret_cast<char*>(p) + bytes); }
 
 struct TeamView {             // private to one team
     float* cx;                // [TW*NC] atom coordinates (grid units), one
@@ -243,8 +262,14 @@ struct TeamView {             // private to one team
 
 __host__ __device__ inline size_t align16(size_t x) { return (x + 15) & ~size_t(15); }
 
-__host__ __device__ inline size_t shared_bytes_for(int T, int P, bool pairs_in_lds) {
-    size_t s = pairs_in_lds ? (size_t)P * (sizeof(PairA) + sizeof(PairB)) : 0;
+// Records from one step of the pair loop to the next.  In LDS the two halves
+// of a step's TW records follow each other (TW PairA, then TW PairB), so that
+// one address register reaches both, at a fixed offset.
+template <int TW, bool PL>
+constexpr int pair_stride = PL ? 2 * TW : TW;
+
+__host__ __device__ inline size_t shared_bytes_for(int TW, int T, int P, bool pairs_in_lds) {
+    size_t s = pairs_in_lds ? (size_t)padded_pairs(P, TW) * (sizeof(PairA) + sizeof(PairB)) : 0;
     s += (size_t)T * (sizeof(float4) * 2 + sizeof(int2));
     return align16(s);
 }
@@ -255,7 +280,7 @@ __host__ __device__ inline size_t team_bytes_for(int natoms_pad, int T) {
 
 // LDS of one workgroup of `threads` threads (threads / TW teams).
 __host__ __device__ inline size_t lds_bytes_for(int TW, int NC, int T, int P, bool pairs_in_lds, int threads = 256) {
-    return shared_bytes_for(T, P, pairs_in_lds) + (size_t)(threads / TW) * team_bytes_for(TW * NC, T);
+    return shared_bytes_for(TW, T, P, pairs_in_lds) + (size_t)(threads / TW) * team_bytes_for(TW * NC, T);
 }
 
 // Stages the shared tables (all threads of the workgroup) and carves the
@@ -267,13 +292,19 @@ DEV void stage(const LigandDev* L, char* lds, SharedView& sv, TeamView& tv) {
     char* p = lds;
     const PairA* gpa = reinterpret_cast<const PairA*>(gbase + L->off_pair_a);
     const PairB* gpb = reinterpret_cast<const PairB*>(gbase + L->off_pair_b);
+    sv.px = reinterpret_cast<const uint32_t*>(gbase + L->off_pair_x);
     if (PL) {
+        const int PP = padded_pairs(P, TW);
         PairA* la = reinterpret_cast<PairA*>(p);
-        PairB* lb = reinterpret_cast<PairB*>(p + (size_t)P * sizeof(PairA));
-        for (int k = threadIdx.x; k < P; k += blockDim.x) { la[k] = gpa[k]; lb[k] = gpb[k]; }
+        PairB* lb = reinterpret_cast<PairB*>(la + TW);
+        for (int k = threadIdx.x; k < PP; k += blockDim.x) {
+            const int at = k / TW * pair_stride<TW, true> + k % TW;
+            la[at] = gpa[k];
+            lb[at] = gpb[k];
+        }
         sv.pa = la;
         sv.pb = lb;
-        p += (size_t)P * (sizeof(PairA) + sizeof(PairB));
+        p += (size_t)PP * (sizeof(PairA) + sizeof(PairB));
     } else {
         sv.pa = gpa;
         sv.pb = gpb;
@@ -287,7 +318,7 @@ DEV void stage(const LigandDev* L, char* lds, SharedView& sv, TeamView& tv) {
     for (int k = threadIdx.x; k < T; k += blockDim.x) { tu[k] = gtu[k]; tm[k] = gtm[k]; ta[k] = gta[k]; }
     sv.tor_unit = tu; sv.tor_move = tm; sv.tor_atoms = ta;
     const int npad = TW * NC;
-    char* w = lds + shared_bytes_for(T, P, PL) + (size_t)(threadIdx.x / TW) * team_bytes_for(npad, T);
+    char* w = lds + shared_bytes_for(TW, T, P, PL) + (size_t)(threadIdx.x / TW) * team_bytes_for(npad, T);
     tv.cx = reinterpret_cast<float*>(w); w += align16((size_t)npad * 4);
     tv.cy = reinterpret_cast<float*>(w); w += align16((size_t)npad * 4);
     tv.cz = reinterpret_cast<float*>(w); w += align16((size_t)npad * 4);
@@ -525,60 +556,57 @@ DEV float gather_finish(const GridDev& G, float3 c, float q, const Gather<MF>& g
 // The cutoff tests select terms instead of branching: over a team's pairs
 // both ranges are almost always present, so branches would only add mask
 // handling.  Adding the zero of an excluded term leaves the sum unchanged.
-// rdist = 1 / (distance in grid units), inv_sp = 1 / spacing: 1/r in A is
-// their product unless r is clamped at elec_min_distance.
+// dist = distance in grid units, rdist = 1 / dist, inv_sp = 1 / spacing: 1/r in
+// A is rdist * inv_sp unless r is clamped at elec_min_distance.  Every fused
+// multiply-add is written out, so all kernels round alike.
 template <bool GRAD>
-DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, float ad, float rdist, float inv_sp,
-                      float& dedr) {
+DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, const uint32_t* px, float spacing,
+                      float dist, float rdist, float inv_sp, float& dedr) {
+#pragma clang fp contract(off)
     // vdW / H-bond with smoothing, r < 8 A: with qm = sd^-m and qn = sd^-n,
     // E = AC qm - BD qn and dE/dsd = -(m AC qm - n BD qn) / sd.  sd^-12 is one
     // reciprocal of sd^12 (a few ulp; the 12th power of 1/sd would carry up to
     // 12 ulp), and sd^-n = sd^-12 sd^(12-n)
-    const float delta = pb.reqm - ad;
-    const float sd = (fabsf(delta) >= ls.half_smooth) ? ad + copysignf(ls.half_smooth, delta) : pb.reqm;
-    const uint32_t fl = pa.flags;
-    const uint32_t nexp = (fl >> 8) & 0xffu;
-    const float q = fast_rcp(sd);
+    const float ad = dist * spacing;
+    const float delta = fmaf(-spacing, dist, pb.reqm);
+    const float sd = (fabsf(delta) >= ls.half_smooth) ? fmaf(spacing, dist, copysignf(ls.half_smooth, delta)) : pb.reqm;
     const float r2 = sd * sd, r4 = r2 * r2, r6 = r4 * r2;
-    float qm = fast_rcp(r6 * r6);                     // m = 12
-    float qn = qm * (nexp == 6u ? r6 : r2);           // n = 6 or 10
-    float fn = (float)nexp;
-    bool general = false;
+    const float qm = fast_rcp(r6 * r6);               // m = 12
+    const float qn = qm * (pa.fn == 6.0f ? r6 : r2);  // n = 6 or 10
+    const float q = GRAD ? fast_rcp(sd) : 0.0f;
+    const float am = pa.ac * qm, bn = pa.bd * qn;
+    float evdw = fmaf(pa.ac, qm, -bn);
+    float dvdw = GRAD ? fmaf(bn, pa.fn, -(12.0f * am)) * q : 0.0f;
     if (__builtin_expect(ls.any_general, 0)) {        // other exponents (modified pairs): rare,
-        if (!(fl & (1u << 17))) {                     // kept off the common path
-            general = true;
+        const uint32_t fl = *px;                      // kept off the common path
+        if (!(fl & kPairFast)) {
+            const float fm = (float)(fl & 0xffu);
             const float l2 = __builtin_amdgcn_logf(sd);
-            qm = __builtin_amdgcn_exp2f(-(float)(fl & 0xffu) * l2);
-            qn = __builtin_amdgcn_exp2f(-fn * l2);
+            const float gm = __builtin_amdgcn_exp2f(-fm * l2);
+            const float ga = pa.ac * gm, gb = pa.bd * __builtin_amdgcn_exp2f(-pa.fn * l2);
+            evdw = fmaf(pa.ac, gm, -gb);
+            if (GRAD) dvdw = fmaf(gb, pa.fn, -(fm * ga)) * q;
         }
     }
-    const float am = pa.ac * qm, bn = pa.bd * qn;
-    const float evdw = am - bn;
     // electrostatics and desolvation, r < 20.48 A, r clamped at elec_min_distance:
     // 1/max(r, r_min) = min(1/r, 1/r_min)
-    const float d = fmaxf(ad, ls.elec_min);
+    const float d = max_s(ad, ls.elec_min);
     const float d2 = d * d;
-    const float desolv = pb.dsol * (ls.coeff_desolv * (12.96f - 0.1063f * d2 * (1.0f - 0.001947f * d2)) *
-                                    fast_rcp(12.96f + d2 * (0.4137f + d2 * (0.00357f + 0.000112f * d2))));
-    const float ds = d + 1.26366f;
-    const float rds = fast_rcp(ds);
+    const float num = fmaf(-0.1063f * d2, fmaf(-0.001947f, d2, 1.0f), 12.96f);
+    const float den = fmaf(d2, fmaf(d2, fmaf(0.000112f, d2, 0.00357f), 0.4137f), 12.96f);
+    const float desolv = pb.dsol * (ls.coeff_desolv * num * fast_rcp(den));
+    const float rds = fast_rcp(d + 1.26366f);
     const float rds2 = rds * rds;
-    const float diel = 1.10859f * rds2 + 0.010358f;
-    const float rd = fminf(rdist * inv_sp, ls.inv_elec_min);
+    const float diel = fmaf(1.10859f, rds2, 0.010358f);
+    const float rd = min_s(rdist * inv_sp, ls.inv_elec_min);
     const float es = pb.cq * rd;
-    const float eel = diel * es + desolv;
+    const float eel = fmaf(es, diel, desolv);
     const bool in8 = ad < 8.0f, in20 = ad < 20.48f;
-    float e = pb.g * ad;                              // CG-G0 bond term, G = 50 (0 for other pairs)
-    e += in8 ? evdw : 0.0f;
-    e += in20 ? eel : 0.0f;
+    // CG-G0 bond term, G = 50 (0 for other pairs)
+    const float e = fmaf(pb.g, ad, in8 ? evdw : 0.0f) + (in20 ? eel : 0.0f);
     if (GRAD) {
-        const float mam = general ? (float)(fl & 0xffu) * am : 12.0f * am;
-        const float dvdw = (fn * bn - mam) * q;
-        const float del = -es * rd * diel - es * 2.21718f * rds2 * rds - 0.0771605f * d * desolv;
-        float g = pb.g;
-        g += in8 ? dvdw : 0.0f;
-        g += in20 ? del : 0.0f;
-        dedr = g;
+        const float del = fmaf(-0.0771605f * d, desolv, fmaf(rds, es * -2.21718f * rds2, -(es * rd * diel)));
+        dedr = pb.g + (in8 ? dvdw : 0.0f) + (in20 ? del : 0.0f);
     } else {
         dedr = 0.f;
     }
@@ -592,7 +620,7 @@ DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, fl
 //                 receives d E / d gene (lane + TW j), 0 beyond the genes.
 // All lanes of the wavefront must call it together (uniform control flow).
 // ---------------------------------------------------------------------------
-template <int TW, int NC, int MF, bool GRAD>
+template <int TW, int NC, int MF, bool PL, bool GRAD>
 DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float (&grad)[64 / TW]) {
     using TM = Team<TW>;
     const LigandDev* L = X.L;
@@ -600,7 +628,7 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
     const TeamView& tv = X.tv;
     const SharedView& sv = X.sv;
     const int tl = TM::lane();
-    const int T = X.ls.T, P = X.ls.P, NG = X.ls.NG;
+    const int T = X.ls.T, NG = X.ls.NG;
     const bool has_lig = X.ls.has_lig;
     (void)L;
 
@@ -624,24 +652,41 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
 
     const float spacing = G.spacing;
     float e = 0.f;
-    for (int p = tl; p < P; p += TW) {
-        const PairA pa = sv.pa[p];
-        const PairB pb = sv.pb[p];
-        const int i = (int)(pa.ij & 0xffffu), j = (int)(pa.ij >> 16);
-        const float sx = tv.cx[i] - tv.cx[j], sy = tv.cy[i] - tv.cy[j], sz = tv.cz[i] - tv.cz[j];
-        const float d2g = sx * sx + sy * sy + sz * sz;
+    const PairA* ra = sv.pa + tl;
+    const PairB* rb = sv.pb + tl;
+    const uint32_t* rx = sv.px + tl;
+    // Every lane has a record in every step (padding), so the loop count is
+    // uniform: no execution masks, and the counter is scalar.  With the atoms
+    // kept as byte offsets, the exponent as a float, the two halves of a step
+    // behind one address and the bounds taken by max_s / min_s, a step is 91
+    // VALU and 8 SALU instructions (105 and 15 with counted lanes, packed
+    // indices and library fmaxf / fminf): Solis-Wets nrun 20 on the 30-atom
+    // ligand 95.6 -> 89.5 ms a docking, ADADELTA nrun 50 on 54 atoms 222.8 ->
+    // 218.0 ms, ADADELTA nrun 100 on 30 atoms 389.2 -> 386.2 ms.
+    const int steps = (X.ls.P + TW - 1) / TW;
+#pragma unroll 1
+    for (int k = 0; k < steps; ++k) {
+        const PairA pa = *ra;
+        const PairB pb = *rb;
+        const uint32_t io = pa.ij & 0xffffu, jo = pa.ij >> 16;
+        const float sx = *at(tv.cx, io) - *at(tv.cx, jo), sy = *at(tv.cy, io) - *at(tv.cy, jo),
+                    sz = *at(tv.cz, io) - *at(tv.cz, jo);
+        const float d2g = fmaf(sz, sz, fmaf(sx, sx, sy * sy));
         const float rdist = fast_rsq(d2g);            // one transcendental for r and 1/r
         const float dist = d2g * rdist;
         float dedr;
-        e += pair_energy<GRAD>(X.ls, pa, pb, dist * spacing, rdist, G.inv_spacing, dedr);
+        e += pair_energy<GRAD>(X.ls, pa, pb, rx, spacing, dist, rdist, G.inv_spacing, dedr);
         if (GRAD) {
             // TERMSCALE * s * gdd with the power-of-two scale folded into gdd:
             // the same rounded product
-            const float gdd = kTermScale * (-dedr * rdist);
+            const float gdd = dedr * rdist * -kTermScale;
             const int ix = quant(sx * gdd), iy = quant(sy * gdd), iz = quant(sz * gdd);
-            lds_sub(&tv.fx[i], ix); lds_sub(&tv.fy[i], iy); lds_sub(&tv.fz[i], iz);
-            atomicAdd(&tv.fx[j], ix); atomicAdd(&tv.fy[j], iy); atomicAdd(&tv.fz[j], iz);
+            lds_sub(at(tv.fx, io), ix); lds_sub(at(tv.fy, io), iy); lds_sub(at(tv.fz, io), iz);
+            atomicAdd(at(tv.fx, jo), ix); atomicAdd(at(tv.fy, jo), iy); atomicAdd(at(tv.fz, jo), iz);
         }
+        ra += pair_stride<TW, PL>;
+        rb += pair_stride<TW, PL>;
+        rx += TW;
     }
     int3 fi[NC];
 #pragma unroll
@@ -759,7 +804,7 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
 // derivatives, used once per FIRE search (calcgradient.cl:109-1003).  Forces
 // are float; intra forces use LDS float atomics of one team.
 // ---------------------------------------------------------------------------
-template <int TW, int NC, int MF>
+template <int TW, int NC, int MF, bool PL>
 DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float (&grad)[64 / TW]) {
     using TM = Team<TW>;
     const LigandDev* L = X.L;
@@ -824,10 +869,11 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
     const float half_smooth = X.ls.half_smooth;
     const float DA = -8.5525f, DB = 78.4f - (-8.5525f), DK = 7.7839f;
     const float DBH = DB * 0.003627f, DBHK = DBH * DK;
-    for (int p = tl; p < P; p += TW) {
-        const PairA pa = sv.pa[p];
-        const PairB pb = sv.pb[p];
-        const int i = (int)(pa.ij & 0xffffu), j = (int)(pa.ij >> 16);
+    for (int p = tl, r = tl; p < P; p += TW, r += pair_stride<TW, PL>) {
+        const PairA pa = sv.pa[r];
+        const PairB pb = sv.pb[r];
+        const uint32_t fl = sv.px[p];
+        const int i = (int)(pa.ij & 0xffffu) >> 2, j = (int)(pa.ij >> 18);
         const float sx = tv.cx[i] - tv.cx[j], sy = tv.cy[i] - tv.cy[j], sz = tv.cz[i] - tv.cz[j];
         const float dist = sqrtf(sx * sx + sy * sy + sz * sz);
         float d = dist * spacing;
@@ -835,7 +881,7 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
         if (d <= pb.reqm - half_smooth) sd = d + half_smooth;
         else if (d < pb.reqm + half_smooth) sd = pb.reqm;
         else sd = d - half_smooth;
-        const int m = (int)(pa.flags & 0xffu), n = (int)((pa.flags >> 8) & 0xffu);
+        const int m = (int)(fl & 0xffu), n = (int)((fl >> 8) & 0xffu);
         float pg = 0.f;
         if (d < 8.0f) {
             pg += (-(float)m * pa.ac) / powf(sd, (float)(m + 1));
@@ -850,7 +896,7 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
             pg += -pb.cq * (upper / lower);
             pg += pb.dsol * X.ls.coeff_desolv * -0.077160f * d * __expf(-0.038580f * d * d);
         }
-        if (pa.flags & (1u << 16)) pg += 50.0f;
+        if (fl & kPairCgG0) pg += 50.0f;
         const float fx = pg * (-sx / dist), fy = pg * (-sy / dist), fz = pg * (-sz / dist);
         atomicAdd(&ffx[i], -fx); atomicAdd(&ffy[i], -fy); atomicAdd(&ffz[i], -fz);
         atomicAdd(&ffx[j], fx); atomicAdd(&ffy[j], fy); atomicAdd(&ffz[j], fz);

@@ -305,8 +305,10 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
     hd.off_tor_unit = take(sizeof(float4) * (T ? T : 1));
     hd.off_tor_move = take(sizeof(float4) * (T ? T : 1));
     hd.off_tor_atoms = take(sizeof(int2) * (T ? T : 1));
-    hd.off_pair_a = take(sizeof(PairA) * (P ? P : 1));
-    hd.off_pair_b = take(sizeof(PairB) * (P ? P : 1));
+    const int PP = padded_pairs(P, kPairPad);
+    hd.off_pair_a = take(sizeof(PairA) * (P ? PP : 1));
+    hd.off_pair_b = take(sizeof(PairB) * (P ? PP : 1));
+    hd.off_pair_x = take(sizeof(uint32_t) * (P ? PP : 1));
     hd.off_type_ds = take(sizeof(float2) * NT);
     hd.total_bytes = (uint32_t)off;
     blob.assign(off, 0);
@@ -348,6 +350,7 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
     for (int t = 0; t < NT; ++t) tds[t] = make_float2(L->ds_s[t], L->ds_v[t]);
     PairA* pra = reinterpret_cast<PairA*>(blob.data() + hd.off_pair_a);
     PairB* prb = reinterpret_cast<PairB*>(blob.data() + hd.off_pair_b);
+    uint32_t* prx = reinterpret_cast<uint32_t*>(blob.data() + hd.off_pair_x);
     for (int q = 0; q < P; ++q) {
         const int p = order[q];
         PairA& ra = pra[q];
@@ -361,8 +364,9 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
         bool cgg0 = (r1 == 24 && r2 == 25) || (r1 == 25 && r2 == 24);   // ATYPE_CG_IDX / ATYPE_G0_IDX
         bool fast = (m == 12) && (n == 6 || n == 10);
         if (!fast) hd.any_general = 1;
-        ra.ij = (uint32_t)i | ((uint32_t)j << 16);
-        ra.flags = m | (n << 8) | ((uint32_t)cgg0 << 16) | ((uint32_t)fast << 17);
+        ra.ij = (uint32_t)(4 * i) | ((uint32_t)(4 * j) << 16);
+        ra.fn = (float)n;
+        prx[q] = m | (n << 8) | (cgg0 ? kPairCgG0 : 0u) | (fast ? kPairFast : 0u);
         ra.ac = L->vw_ac[idx];
         ra.bd = L->vw_bd[idx];
         rb.reqm = L->reqm_ab[idx];
@@ -371,6 +375,13 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
         rb.dsol = (L->ds_s[t1] + ep->qasp * std::fabs(q1)) * L->ds_v[t2] +
                   (L->ds_s[t2] + ep->qasp * std::fabs(q2)) * L->ds_v[t1];   // calcenergy.cl:488-491
         rb.g = cgg0 ? 50.0f : 0.0f;                             // calcenergy.cl:452-458, G = 50
+    }
+    for (int q = P; P && q < PP; ++q) {   // padding (kPairPad): a real pair's geometry, no terms
+        const int p = (q - P) % P;
+        pra[q].ij = pra[p].ij;
+        pra[q].fn = 6.0f;
+        prb[q].reqm = prb[p].reqm;
+        prx[q] = 12u | (6u << 8) | kPairFast;
     }
     std::memcpy(blob.data(), &hd, sizeof(hd));
     return ADGPU_OK;

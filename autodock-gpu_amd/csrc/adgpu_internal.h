@@ -16,10 +16,12 @@ constexpr int kGenes = ADGPU_GENOTYPE_STRIDE;
 // One intramolecular pair, precomputed on the host from the reference's
 // per-type tables (the lookups of calcenergy.cl:397-536 folded per pair), in
 // two 16-byte halves stored as separate arrays so that consecutive lanes read
-// consecutive 16-byte records (no LDS bank conflicts).
+// consecutive 16-byte records (no LDS bank conflicts).  Atoms and exponent
+// are kept in the form the pair loop uses (byte offsets into its coordinate
+// arrays, a float), so that it spends no instruction on unpacking them.
 struct __attribute__((aligned(16))) PairA {
-    uint32_t ij;      // atom1 | atom2 << 16
-    uint32_t flags;   // m | n << 8 | (CG-G0 bond) << 16 | (fast 12-6 / 12-10 form) << 17
+    uint32_t ij;      // 4 * atom1 | (4 * atom2) << 16
+    float fn;         // exponent n of the attractive term
     float ac;         // VWpars_AC of the type pair
     float bd;         // VWpars_BD
 };
@@ -29,6 +31,15 @@ struct __attribute__((aligned(16))) PairB {
     float dsol;       // (S1 + qasp|q1|) V2 + (S2 + qasp|q2|) V1
     float g;          // CG-G0 bond constant G: 50 for a CG-G0 pair, else 0
 };
+// PairX flags: m | n << 8 | (CG-G0 bond) << 16 | (12-6 / 12-10 form) << 17.
+constexpr uint32_t kPairCgG0 = 1u << 16, kPairFast = 1u << 17;
+
+// The pair arrays are padded to a multiple of the widest team, so that every
+// lane of every team takes part in every step of the pair loop.  A padding
+// record repeats the atoms and the optimum distance of a real pair with all
+// coefficients zero: it adds zero (or NaN where the real pair's term is NaN).
+constexpr int kPairPad = 64;
+__host__ __device__ inline int padded_pairs(int pairs, int to) { return (pairs + to - 1) / to * to; }
 
 // Everything the kernels need about one ligand, in one device allocation.
 // Offsets are in bytes from the start of the block.
@@ -43,10 +54,11 @@ struct LigandDev {
     uint32_t off_tor_unit;    // float4 [T]  unit vector
     uint32_t off_tor_move;    // float4 [T]  moving vector
     uint32_t off_tor_atoms;   // int2   [T]  bond atoms
-    uint32_t off_pair_a;      // PairA[P]
-    uint32_t off_pair_b;      // PairB[P]
+    uint32_t off_pair_a;      // PairA[P padded to kPairPad]
+    uint32_t off_pair_b;      // PairB[P padded]
+    uint32_t off_pair_x;      // uint32 [P padded] flags (PairX)
     uint32_t off_type_ds;     // float2 [num_atypes] (dspars_S, dspars_V) per ligand type (FP64 re-scoring)
-    uint32_t total_bytes, pad6, pad7;
+    uint32_t total_bytes, pad6;
 };
 
 struct GridDev {

@@ -20,12 +20,12 @@ __global__ ADGPU_GROUP_KERNEL void k_eval_poses(Launch a) {
 #pragma unroll
     for (int j = 0; j < GPL; ++j) gene[j] = a.in_geno[(size_t)id * kGenes + tl + TW * j];
     if (a.mode == ADGPU_EVAL_GRADIENT) {
-        float_gradient<TW, NC, MF>(X, gene, grad);
+        float_gradient<TW, NC, MF, PL>(X, gene, grad);
     } else if (a.mode == ADGPU_EVAL_ENERGRAD) {
-        const float e = evaluate<TW, NC, MF, true>(X, gene, grad);
+        const float e = evaluate<TW, NC, MF, PL, true>(X, gene, grad);
         if (live && tl == 0 && a.out_e) a.out_e[id] = e;
     } else {
-        const float e = evaluate<TW, NC, MF, false>(X, gene, grad);
+        const float e = evaluate<TW, NC, MF, PL, false>(X, gene, grad);
         if (live && tl == 0 && a.out_e) a.out_e[id] = e;
         return;
     }

@@ -19,7 +19,7 @@ __global__ ADGPU_GROUP_KERNEL void k_initpop(Launch a) {
     float gene[GPL], grad[GPL];
 #pragma unroll
     for (int j = 0; j < GPL; ++j) gene[j] = a.B.pop_cur[(size_t)id * kGenes + tl + TW * j];
-    const float e = evaluate<TW, NC, MF, false>(X, gene, grad);
+    const float e = evaluate<TW, NC, MF, PL, false>(X, gene, grad);
     if (live && tl == 0) { a.B.ene_cur[id] = e; a.B.evals_new[id] = 1; }
 }
 
@@ -42,7 +42,7 @@ __global__ ADGPU_GROUP_KERNEL void k_gen(Launch a) {
     k4_prepare<TW>(a.S, a.B.pop_cur + (size_t)run * pop * kGenes, a.B.ene_cur + (size_t)run * pop, st, ent, it);
     float in[GPL], grad[GPL];
     k4_genes<TW>(it, NG, in);
-    const float e = evaluate<TW, NC, MF, false>(X, in, grad);
+    const float e = evaluate<TW, NC, MF, PL, false>(X, in, grad);
     if (!live) return;
     k4_store<TW>(it, NG, e, a.B.pop_next + (size_t)idx * kGenes, a.B.ene_next + idx, a.B.evals_new + idx, st);
 }

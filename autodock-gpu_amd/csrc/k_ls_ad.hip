@@ -253,7 +253,7 @@ __global__ ADGPU_GROUP_KERNEL void k_ls_ad(Launch a) {
             peek = __hip_atomic_load(&seats[it.cons_fail], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         float g[GPL];
         ++steps;
-        const float e = evaluate<TW, NC, MF, true>(X, it.geno, g);
+        const float e = evaluate<TW, NC, MF, PL, true>(X, it.geno, g);
         // no other team of the wavefront has a search or may still get one from
         // the queue or the ring; a search moves only to a seat older than every
         // seat its wavefront holds, so two half-idle wavefronts merge toward the

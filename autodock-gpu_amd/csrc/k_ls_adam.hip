@@ -58,7 +58,7 @@ __global__ ADGPU_GROUP_KERNEL void k_ls_adam(Launch a) {
         }
         ++steps;
         float g[GPL];
-        const float e = evaluate<TW, NC, MF, true>(X, geno, g);
+        const float e = evaluate<TW, NC, MF, PL, true>(X, geno, g);
         if (!done) {
             const float b1p = 1.0f - powf(b1, 1.0f + (float)iters);
             const float b2p = 1.0f - powf(b2, 1.0f + (float)iters);

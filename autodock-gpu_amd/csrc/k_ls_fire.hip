@@ -31,7 +31,7 @@ __global__ ADGPU_GROUP_KERNEL void k_fire_init(Launch a) {
         const int g = tl + TW * j;
         geno[j] = g < NG ? a.B.pop_next[gi * kGenes + g] : 0.f;
     }
-    float_gradient<TW, NC, MF>(X, geno, grad);
+    float_gradient<TW, NC, MF, PL>(X, geno, grad);
     if (!live) return;
 #pragma unroll
     for (int j = 0; j < GPL; ++j) a.B.ls_grad[(size_t)t * kGenes + tl + TW * j] = grad[j];
@@ -99,7 +99,7 @@ __global__ ADGPU_GROUP_KERNEL void k_ls_fire(Launch a) {
         float cand[GPL], cg[GPL];
 #pragma unroll
         for (int j = 0; j < GPL; ++j) cand[j] = geno[j] + dt * vel[j];
-        const float ce = evaluate<TW, NC, MF, true>(X, cand, cg);
+        const float ce = evaluate<TW, NC, MF, PL, true>(X, cand, cg);
         float pw = 0.f, og = 0.f, ng = 0.f;
 #pragma unroll
         for (int j = 0; j < GPL; ++j) { pw += -cg[j] * vel[j]; og += grad[j] * grad[j]; ng += cg[j] * cg[j]; }

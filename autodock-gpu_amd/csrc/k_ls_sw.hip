@@ -99,7 +99,7 @@ __global__ ADGPU_GROUP_KERNEL void k_ls_sw(Launch a) {
             }
         }
         float grad[GPL];
-        const float ce = evaluate<TW, NC, MF, false>(X, cand, grad);
+        const float ce = evaluate<TW, NC, MF, PL, false>(X, cand, grad);
         if (!done) {
             evals++;
             bool iter_end = false;

@@ -52,6 +52,7 @@ __global__ __launch_bounds__(64) void k_rescore_f64(const LigandDev* L, GridDev 
     const float4* tm = reinterpret_cast<const float4*>(gb + L->off_tor_move);
     const PairA* pa = reinterpret_cast<const PairA*>(gb + L->off_pair_a);
     const PairB* pb = reinterpret_cast<const PairB*>(gb + L->off_pair_b);
+    const uint32_t* px = reinterpret_cast<const uint32_t*>(gb + L->off_pair_x);
     const float2* tds = reinterpret_cast<const float2*>(gb + L->off_type_ds);
     const float* g = geno + (size_t)pose * kGenes;
     const double d2r = (double)kDegToRad;
@@ -118,12 +119,13 @@ __global__ __launch_bounds__(64) void k_rescore_f64(const LigandDev* L, GridDev 
     for (int k = lane; k < P; k += 64) {   // pair terms, calcenergy.cl:397-536
         const PairA A = pa[k];
         const PairB B = pb[k];
-        const int i = (int)(A.ij & 0xffffu), j = (int)(A.ij >> 16);
+        const uint32_t flags = px[k];
+        const int i = (int)(A.ij & 0xffffu) >> 2, j = (int)(A.ij >> 18);
         const double sx = cx[i] - cx[j], sy = cy[i] - cy[j], sz = cz[i] - cz[j];
         const double dist = sqrt(sx * sx + sy * sy + sz * sz) * spacing;
-        double e = ((A.flags >> 16) & 1u) ? 50.0 * dist : 0.0;   // CG-G0 bond term
+        double e = (flags & kPairCgG0) ? 50.0 * dist : 0.0;   // CG-G0 bond term
         if (dist < 8.0) {
-            const int m = (int)(A.flags & 0xffu), nn = (int)((A.flags >> 8) & 0xffu);
+            const int m = (int)(flags & 0xffu), nn = (int)((flags >> 8) & 0xffu);
             const double opt = (double)B.reqm, od = opt - dist;
             const double sd = fabs(od) >= delta_distance ? dist + copysign(delta_distance, od) : opt;
             const double rmn = pow(sd, (double)(m - nn)), rm = pow(sd, (double)(-m));

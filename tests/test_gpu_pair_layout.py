@@ -1,0 +1,62 @@
+"""The pair loop's padded records: pair counts at and around the team widths
+(the last step of the loop, its padding, no pairs at all), other exponents and
+CG-G0 bonds, energies and merged gradients against the FP32 oracle with the
+bars of test_gpu_parity."""
+import copy
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+import adgpu
+import helpers
+import oracle as O
+from adgpu._abi import CLigand
+
+pytestmark = pytest.mark.gpu
+
+
+def _with(case, **kw):
+    t = copy.copy(case.tables)
+    for k, v in kw.items():
+        setattr(t, k, v)
+    cl = CLigand(t)
+    return SimpleNamespace(**{**vars(case), "tables": t, "cl": cl, "orc": O.Oracle(case.cg, cl, case.ep)})
+
+
+def _forms(c1):
+    pairs = np.asarray(c1.tables.pairs).reshape(-1, 2)
+    for n in (0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 129):
+        yield _with(c1, pairs=pairs[:n].reshape(-1))
+    exps = np.array(c1.tables.vw_exp).copy()
+    exps[1::3] = (9 << 8) + 7
+    yield _with(c1, vw_exp=exps)                     # exponents other than 12-6 / 12-10
+    types = np.array(c1.tables.atype_reqm).copy()
+    types[:2] = (24, 25)
+    yield _with(c1, atype_reqm=types)                # CG-G0 bond terms
+
+
+@pytest.mark.parametrize("width", [16, 32, 64])
+def test_padded_pairs(gpu_ctx, c1, width):
+    mid = gpu_ctx.maps_upload(c1.packed, c1.size, c1.maps.num_map_atypes, c1.spacing)
+    gpu_ctx.set_team_width(width)
+    try:
+        for case in _forms(c1):
+            lid = gpu_ctx.ligand_upload(case.tables, case.ep)
+            poses = helpers.poses_for(case, 120, seed=77)
+            e, g = gpu_ctx.eval_poses(mid, lid, poses, adgpu.EVAL_ENERGRAD)
+            helpers.check_energies(case.orc, poses, e, edge_share=0.05)
+            e2, _ = gpu_ctx.eval_poses(mid, lid, poses, adgpu.EVAL_ENERGY)
+            helpers.check_energies(case.orc, poses, e2, e_ref=e, edge_share=0.05)
+            well = [0, 1, 2] + list(range(6, case.ng))
+            quantum = np.array([helpers.gene_quantum(case, k) for k in range(case.ng)])
+            off = 0
+            for p, row in zip(poses, g):
+                _, go = case.orc.energrad32(p, True)
+                off += int((np.abs(row[:case.ng] - go)[well] > (1e-4 * np.abs(go) + 4 * quantum)[well]).sum())
+            assert off <= 0.002 * len(poses) * len(well)
+            assert np.all(g[:, case.ng:] == 0.0)
+            gpu_ctx.ligand_release(lid)
+    finally:
+        gpu_ctx.set_team_width(0)
+        gpu_ctx.maps_release(mid)
