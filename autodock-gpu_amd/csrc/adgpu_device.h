@@ -32,12 +32,12 @@
 namespace adgpu {
 
 #define DEV __device__ __forceinline__
-// 256-thread workgroups; at least 4 wavefronts per SIMD (<= 128 VGPRs)
+// Workgroups of up to 1024 threads; at least 4 wavefronts per SIMD (<= 128 VGPRs)
 // Waves per SIMD the register budget is sized for (4: at most 128 VGPRs).
 #ifndef ADGPU_WAVES_PER_EU
 #define ADGPU_WAVES_PER_EU 4
 #endif
-#define ADGPU_GROUP_KERNEL __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADGPU_WAVES_PER_EU)))
+#define ADGPU_GROUP_KERNEL __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(ADGPU_WAVES_PER_EU)))
 
 // common/calcenergy_basic.h
 constexpr float kDegToRad = 0.0174533f;
@@ -236,7 +236,7 @@ DEV float4 load_pt<ADGPU_MAP_BF16>(const void* base, uint32_t idx) {
 struct SharedView {           // staged once per workgroup
     const PairA* pa;          // LDS (or global when the pairs do not fit): record p of step k is
     const PairB* pb;          //   [k * pair_stride<TW, PL> + lane] of both
-    const uint32_t* px;       // flags, global (read for exponents other than 12-6 / 12-10)
+    const PairX* px;          // global (rarely read)
     const float4* tor_unit;
     const float4* tor_move;
     const int2* tor_atoms;
@@ -247,16 +247,17 @@ template <class V>
 DEV V* at(V* p, uint32_t bytes) { return reinterpret_cast<V*>(reinterpret_cast<char*>(p) + bytes); }
 
 struct TeamView {             // private to one team
-    float* cx;                // [TW*NC] atom coordinates (grid units), one
+    float* cx;                // [slot_array] atom coordinates (grid units), one
     float* cy;                //   array per axis: lanes reading different
     float* cz;                //   atoms hit different banks
-    int* fx;                  // [TW*NC] int32 fixed-point pair forces
+    int* fx;                  // [slot_array] int32 fixed-point pair forces
     int* fy;
     int* fz;
     float4* tq;               // [T] torsion quaternions
     float4* tax;              // [T] torsion axes (gradient)
     float4* tref;             // [T] torsion reference atoms (gradient)
-    int* gi;                  // [T] torsion gene gradients (int fixed point)
+    int* gi;                  // [T][4] torsion gene gradients (int fixed point), in
+                              //   four parts: lanes add to the part of their index mod 4
     float* pg;                // [12] genes 0..5, sin/cos of phi, theta, rot/2
 };
 
@@ -274,13 +275,13 @@ __host__ __device__ inline size_t shared_bytes_for(int TW, int T, int P, bool pa
     return align16(s);
 }
 
-__host__ __device__ inline size_t team_bytes_for(int natoms_pad, int T) {
-    return 6 * align16((size_t)natoms_pad * 4) + (size_t)T * 48 + align16((size_t)T * 4) + 48;
+__host__ __device__ inline size_t team_bytes_for(int TW, int NC, int T) {
+    return 6 * (size_t)slot_array(TW, NC) * 4 + (size_t)T * 48 + (size_t)T * 16 + 48;
 }
 
 // LDS of one workgroup of `threads` threads (threads / TW teams).
 __host__ __device__ inline size_t lds_bytes_for(int TW, int NC, int T, int P, bool pairs_in_lds, int threads = 256) {
-    return shared_bytes_for(TW, T, P, pairs_in_lds) + (size_t)(threads / TW) * team_bytes_for(TW * NC, T);
+    return shared_bytes_for(TW, T, P, pairs_in_lds) + (size_t)(threads / TW) * team_bytes_for(TW, NC, T);
 }
 
 // Stages the shared tables (all threads of the workgroup) and carves the
@@ -290,9 +291,9 @@ DEV void stage(const LigandDev* L, char* lds, SharedView& sv, TeamView& tv) {
     const char* gbase = reinterpret_cast<const char*>(L);
     const int T = L->num_rotbonds, P = L->num_pairs;
     char* p = lds;
-    const PairA* gpa = reinterpret_cast<const PairA*>(gbase + L->off_pair_a);
+    const PairA* gpa = reinterpret_cast<const PairA*>(gbase + L->off_pair_a[slot_copies(TW, NC) - 1]);
     const PairB* gpb = reinterpret_cast<const PairB*>(gbase + L->off_pair_b);
-    sv.px = reinterpret_cast<const uint32_t*>(gbase + L->off_pair_x);
+    sv.px = reinterpret_cast<const PairX*>(gbase + L->off_pair_x);
     if (PL) {
         const int PP = padded_pairs(P, TW);
         PairA* la = reinterpret_cast<PairA*>(p);
@@ -317,20 +318,21 @@ DEV void stage(const LigandDev* L, char* lds, SharedView& sv, TeamView& tv) {
     const int2* gta = reinterpret_cast<const int2*>(gbase + L->off_tor_atoms);
     for (int k = threadIdx.x; k < T; k += blockDim.x) { tu[k] = gtu[k]; tm[k] = gtm[k]; ta[k] = gta[k]; }
     sv.tor_unit = tu; sv.tor_move = tm; sv.tor_atoms = ta;
-    const int npad = TW * NC;
-    char* w = lds + shared_bytes_for(TW, T, P, PL) + (size_t)(threadIdx.x / TW) * team_bytes_for(npad, T);
-    tv.cx = reinterpret_cast<float*>(w); w += align16((size_t)npad * 4);
-    tv.cy = reinterpret_cast<float*>(w); w += align16((size_t)npad * 4);
-    tv.cz = reinterpret_cast<float*>(w); w += align16((size_t)npad * 4);
-    tv.fx = reinterpret_cast<int*>(w); w += align16((size_t)npad * 4);
-    tv.fy = reinterpret_cast<int*>(w); w += align16((size_t)npad * 4);
-    tv.fz = reinterpret_cast<int*>(w); w += align16((size_t)npad * 4);
+    char* w = lds + shared_bytes_for(TW, T, P, PL) + (size_t)(threadIdx.x / TW) * team_bytes_for(TW, NC, T);
+    constexpr int kArray = slot_array(TW, NC);
+    tv.cx = reinterpret_cast<float*>(w);
+    tv.cy = tv.cx + kArray;
+    tv.cz = tv.cy + kArray;
+    tv.fx = reinterpret_cast<int*>(tv.cz + kArray);
+    tv.fy = tv.fx + kArray;
+    tv.fz = tv.fy + kArray;
+    w += 6 * (size_t)kArray * 4;
     tv.tq = reinterpret_cast<float4*>(w);
     tv.tax = tv.tq + T;
     tv.tref = tv.tax + T;
     w += (size_t)T * 48;
     tv.gi = reinterpret_cast<int*>(w);
-    w += align16((size_t)T * 4);
+    w += (size_t)T * 16;
     tv.pg = reinterpret_cast<float*>(w);
     __syncthreads();
 }
@@ -344,6 +346,8 @@ struct Atoms {
     float q[NC];
     uint32_t mlo[NC], mhi[NC];
     uint32_t mapoff[NC];      // map index * g3
+    uint32_t slot[NC];        // byte offset of the atom's first copy in the slot arrays
+    uint32_t copy;            // bytes from there to its second copy
     bool valid[NC], ign[NC], lig[NC];
 
     DEV void load(const LigandDev* L, const GridDev& G) {
@@ -352,10 +356,14 @@ struct Atoms {
         const int4* ai = reinterpret_cast<const int4*>(gb + L->off_atom_info);
         const uint2* am = reinterpret_cast<const uint2*>(gb + L->off_atom_mask);
         const int tl = Team<TW>::lane();
+        const int stride = slot_stride(L->num_atoms);
+        copy = (uint32_t)stride * 4u;
 #pragma unroll
         for (int k = 0; k < NC; ++k) {
             int a = tl + TW * k;
             valid[k] = a < L->num_atoms;
+            // without an atom: the first slot behind them, which no pair names
+            slot[k] = 4u * (uint32_t)(valid[k] ? a : slot_copies(TW, NC) == 2 ? stride - 16 : TW * NC);
             int aa = valid[k] ? a : 0;
             float4 r = ar[aa];
             int4 inf = ai[aa];
@@ -463,7 +471,6 @@ DEV Pose read_pose(const TeamView& tv, bool has_ligand) {
 template <int TW, int NC>
 DEV void compute_coords(const SharedView& sv, const TeamView& tv, const Atoms<TW, NC>& A, const Pose& P,
                         float3 (&c)[NC]) {
-    const int tl = Team<TW>::lane();
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
         float3 v = A.ref[k];
@@ -482,9 +489,11 @@ DEV void compute_coords(const SharedView& sv, const TeamView& tv, const Atoms<TW
             v = make_float3(r.x + P.mv.x, r.y + P.mv.y, r.z + P.mv.z);
         }
         c[k] = v;
-        tv.cx[tl + TW * k] = v.x;
-        tv.cy[tl + TW * k] = v.y;
-        tv.cz[tl + TW * k] = v.z;
+#pragma unroll
+        for (int copy = 0; copy < slot_copies(TW, NC); ++copy) {
+            const uint32_t o = A.slot[k] + copy * A.copy;
+            *at(tv.cx, o) = v.x; *at(tv.cy, o) = v.y; *at(tv.cz, o) = v.z;
+        }
     }
 }
 
@@ -560,7 +569,7 @@ DEV float gather_finish(const GridDev& G, float3 c, float q, const Gather<MF>& g
 // A is rdist * inv_sp unless r is clamped at elec_min_distance.  Every fused
 // multiply-add is written out, so all kernels round alike.
 template <bool GRAD>
-DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, const uint32_t* px, float spacing,
+DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, const PairX* px, float spacing,
                       float dist, float rdist, float inv_sp, float& dedr) {
 #pragma clang fp contract(off)
     // vdW / H-bond with smoothing, r < 8 A: with qm = sd^-m and qn = sd^-n,
@@ -578,7 +587,7 @@ DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, co
     float evdw = fmaf(pa.ac, qm, -bn);
     float dvdw = GRAD ? fmaf(bn, pa.fn, -(12.0f * am)) * q : 0.0f;
     if (__builtin_expect(ls.any_general, 0)) {        // other exponents (modified pairs): rare,
-        const uint32_t fl = *px;                      // kept off the common path
+        const uint32_t fl = px->flags;                // kept off the common path
         if (!(fl & kPairFast)) {
             const float fm = (float)(fl & 0xffu);
             const float l2 = __builtin_amdgcn_logf(sd);
@@ -635,8 +644,13 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
     gene_trig<TW>(X.ls, sv, tv, gene);
     if (GRAD) {
 #pragma unroll
-        for (int k = 0; k < NC; ++k) { tv.fx[tl + TW * k] = 0; tv.fy[tl + TW * k] = 0; tv.fz[tl + TW * k] = 0; }
-        for (int t = tl; t < T; t += TW) tv.gi[t] = 0;
+        for (int k = 0; k < NC; ++k)
+#pragma unroll
+            for (int copy = 0; copy < slot_copies(TW, NC); ++copy) {
+                const uint32_t o = X.A.slot[k] + copy * X.A.copy;
+                *at(tv.fx, o) = 0; *at(tv.fy, o) = 0; *at(tv.fz, o) = 0;
+            }
+        for (int t = tl; t < T; t += TW) reinterpret_cast<int4*>(tv.gi)[t] = make_int4(0, 0, 0, 0);
     }
     wave_sync();
     const Pose pose = read_pose(tv, has_lig);
@@ -654,7 +668,7 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
     float e = 0.f;
     const PairA* ra = sv.pa + tl;
     const PairB* rb = sv.pb + tl;
-    const uint32_t* rx = sv.px + tl;
+    const PairX* rx = sv.px + tl;
     // Every lane has a record in every step (padding), so the loop count is
     // uniform: no execution masks, and the counter is scalar.  With the atoms
     // kept as byte offsets, the exponent as a float, the two halves of a step
@@ -711,10 +725,14 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
     float sfx = 0.f, sfy = 0.f, sfz = 0.f, tx = 0.f, ty = 0.f, tz = 0.f;
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-        const int a = tl + TW * k;
         F[k] = make_float3(0.f, 0.f, 0.f);
         if (X.A.valid[k]) {
-            int fx = tv.fx[a], fy = tv.fy[a], fz = tv.fz[a];
+            int fx = 0, fy = 0, fz = 0;
+#pragma unroll
+            for (int copy = 0; copy < slot_copies(TW, NC); ++copy) {
+                const uint32_t o = X.A.slot[k] + copy * X.A.copy;
+                fx += *at(tv.fx, o); fy += *at(tv.fy, o); fz += *at(tv.fz, o);
+            }
             if (!X.A.ign[k]) { fx += fi[k].x; fy += fi[k].y; fz += fi[k].z; }
             F[k] = make_float3(kOneOverTermScale * (float)fx, kOneOverTermScale * (float)fy,
                                kOneOverTermScale * (float)fz);
@@ -781,7 +799,7 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
             const float qx = ry * F[k].z - rz * F[k].y, qy = rz * F[k].x - rx * F[k].z,
                         qz = rx * F[k].y - ry * F[k].x;
             const float toa = (ax.x * qx + ax.y * qy + ax.z * qz) * spacing;
-            atomicAdd(&tv.gi[t], quant(kTermScale * toa * kDegToRad));
+            atomicAdd(&tv.gi[4 * t + (tl & 3)], quant(kTermScale * toa * kDegToRad));
         }
     }
     wave_sync();
@@ -791,7 +809,10 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
         const int g = tl + TW * j;
         int iv = 0;
         if (g < 6) iv = ig;
-        else if (g < NG) iv = tv.gi[g - 6];
+        else if (g < NG) {
+            const int4 part = reinterpret_cast<const int4*>(tv.gi)[g - 6];
+            iv = part.x + part.y + part.z + part.w;
+        }
         float gv = kOneOverTermScale * (float)iv;
         if (g >= 3) gv *= conv;
         grad[j] = g < NG ? gv : 0.f;
@@ -822,7 +843,10 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
 
     gene_trig<TW>(X.ls, sv, tv, gene);
 #pragma unroll
-    for (int k = 0; k < NC; ++k) { ffx[tl + TW * k] = 0.f; ffy[tl + TW * k] = 0.f; ffz[tl + TW * k] = 0.f; }
+    for (int k = 0; k < NC; ++k) {
+        const uint32_t o = X.A.slot[k];
+        *at(ffx, o) = 0.f; *at(ffy, o) = 0.f; *at(ffz, o) = 0.f;
+    }
     for (int t = tl; t < T; t += TW) tacc[t] = 0.f;
     wave_sync();
     const Pose pose = read_pose(tv, has_lig);
@@ -872,8 +896,9 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
     for (int p = tl, r = tl; p < P; p += TW, r += pair_stride<TW, PL>) {
         const PairA pa = sv.pa[r];
         const PairB pb = sv.pb[r];
-        const uint32_t fl = sv.px[p];
-        const int i = (int)(pa.ij & 0xffffu) >> 2, j = (int)(pa.ij >> 18);
+        // the pair's atoms in the list's order, first copies: float sums keep their order
+        const uint32_t fl = sv.px[p].flags, atoms = sv.px[p].atoms;
+        const int i = (int)(atoms & 0xffffu), j = (int)(atoms >> 16);
         const float sx = tv.cx[i] - tv.cx[j], sy = tv.cy[i] - tv.cy[j], sz = tv.cz[i] - tv.cz[j];
         const float dist = sqrtf(sx * sx + sy * sy + sz * sz);
         float d = dist * spacing;
@@ -1036,21 +1061,28 @@ struct Shape {
     int tw, nc;
     bool pl;
     size_t lds;
-    int threads;   // workgroup size (64, 128 or 256)
+    int threads;   // workgroup size (64 to 1024)
 };
 
-// Pair records are staged in LDS only while at least three workgroups still
-// fit in a compute unit's 160 KB: beyond that, reading them through L1/L2
-// keeps the four workgroups the registers allow.  Measured (M evals/s, FIRE /
-// ADADELTA): 60 atoms in 64-lane teams, 57 KB in LDS (2 workgroups) 145 / 139
-// against 172 / 167 from memory; 50 atoms in 32-lane teams, 49 KB in LDS (3
-// workgroups) 236 / 204 against 206 / 192 from memory.
-constexpr size_t kLdsBudget = 160 * 1024 / 3;
+// LDS of a compute unit, and the wavefronts that fit on one at the kernels'
+// register budget (four on each of its four SIMDs).
+constexpr size_t kCuLds = 160 * 1024;
+constexpr int kCuWaves = 16;
+constexpr int kCus = 256;
+
+// Wavefronts that workgroups of `threads` threads and `lds` bytes put on a
+// compute unit.
+inline int waves_per_cu(size_t lds, int threads) {
+    const int waves = (int)(kCuLds / (lds ? lds : 1)) * (threads / kWave);
+    return waves < kCuWaves ? waves : kCuWaves;
+}
 
 // Chooses the team width and atom chunks for a ligand: the requested width,
 // else 32-lane teams (two individuals per wavefront) up to 128 atoms and
 // 64-lane teams beyond; 16-lane teams (four per wavefront) only for ligands
-// of at most 32 atoms.  Jobs pass the width fixed when they start.
+// of at most 32 atoms.  Jobs pass the width fixed when they start.  Pair
+// records are staged in LDS while at least 12 wavefronts fit on a compute unit
+// with them; beyond that they are read through L1/L2.
 inline Shape choose_shape(const LigandDev& L, int team_width_hint, int threads = 256) {
     Shape s{};
     s.threads = threads;
@@ -1059,8 +1091,31 @@ inline Shape choose_shape(const LigandDev& L, int team_width_hint, int threads =
     s.tw = tw;
     const int per = (N + tw - 1) / tw;
     s.nc = per <= 1 ? 1 : (per <= 2 ? 2 : 4);
-    s.pl = lds_bytes_for(s.tw, s.nc, L.num_rotbonds, L.num_pairs, true, threads) <= kLdsBudget;
+    s.pl = waves_per_cu(lds_bytes_for(s.tw, s.nc, L.num_rotbonds, L.num_pairs, true, threads), threads) >= 12;
     s.lds = lds_bytes_for(s.tw, s.nc, L.num_rotbonds, L.num_pairs, s.pl, threads);
+    return s;
+}
+
+// Shape of a persistent local-search launch.  All teams of a workgroup share
+// one copy of the pair records, so where a compute unit cannot hold the copies
+// of four 256-thread workgroups, larger workgroups keep the records in LDS at
+// full occupancy: 54 atoms in 64-lane teams, ADADELTA nrun 50, 197 ms a docking
+// with 512 threads, 265 ms with 256 (records through L1/L2).  Not for launches
+// whose searches all fit at once in 256-thread workgroups, which spread them
+// over more compute units (8.5 against 10.2 us an iteration with 16 searches),
+// and not in a server: larger workgroups need half or all of a compute unit
+// free at once, which the launches of other requests seldom leave (24 ligands
+// in 16 slots 0.56 s against 0.50 s).
+inline Shape choose_ls_shape(const LaunchArgs& la, int searches, int threads) {
+    const LigandDev& L = *la.lig_host;
+    const Shape s = choose_shape(L, la.team_hint, threads);
+    const int waves = waves_per_cu(s.lds, threads);
+    if (la.crowded || threads != kGroupThreads || (s.pl && waves == kCuWaves)) return s;
+    if ((int64_t)searches * s.tw / kWave * la.share <= (int64_t)waves * kCus) return s;
+    for (int t = 2 * kGroupThreads; t <= 4 * kGroupThreads; t *= 2) {
+        const Shape w = choose_shape(L, la.team_hint, t);
+        if (w.pl && waves_per_cu(w.lds, t) == kCuWaves) return w;
+    }
     return s;
 }
 

@@ -270,6 +270,43 @@ uint16_t f32_to_bf16(float f) {   // round to nearest even
     return (uint16_t)(r >> 16);
 }
 
+// Chooses the slots of 32 consecutive pairs, which half a wavefront handles in
+// one step (half of them at a time in 16-lane teams): either atom of a pair
+// may be its first (the forces on both are equal and opposite, to the bit)
+// and, with two copies, either copy may stand for each.  Every pair in turn
+// takes the choice whose two banks are least loaded, twice over.  LDS cycles
+// of the six force additions of a wavefront's step by this load model: 65 ->
+// 28 at 30 atoms, 138 -> 42 at 16, 49 -> 25 at 41 (40 with one copy), 28 -> 25
+// at 90 (one copy).
+void spread_slots(int copies, int stride, const PairX* px, PairA* pa) {
+    constexpr int kBanks = 32, kPairs = 32;
+    int load[2][kBanks] = {};                          // cycles of each bank, per atom of the pair
+    uint8_t lanes[2][2 * (ADGPU_MAX_ATOMS + 16)] = {};  // lanes that add to each slot
+    int chosen[kPairs][2];
+    auto put = [&](int r, int slot, int by) {
+        int& m = (lanes[r][slot] += (uint8_t)by, load[r][slot % kBanks]);
+        m += by * (lanes[r][slot] == (by > 0 ? 1 : 0) ? 1 : 2);
+    };
+    auto cost = [&](int r, int slot) {
+        const int c = load[r][slot % kBanks] + (lanes[r][slot] ? 2 : 1);
+        return c * c;
+    };
+    for (int pass = 0; pass < 2; ++pass)
+        for (int k = 0; k < kPairs; ++k) {
+            if (pass) { put(0, chosen[k][0], -1); put(1, chosen[k][1], -1); }
+            const int atom[2] = {(int)(px[k].atoms & 0xffffu), (int)(px[k].atoms >> 16)};
+            int best = -1;
+            for (int o = 0; o < 2 * copies * copies; ++o) {
+                const int a = atom[o & 1] + o / 2 % copies * stride, b = atom[~o & 1] + o / 2 / copies * stride;
+                const int c = cost(0, a) + cost(1, b);
+                if (best < 0 || c < best) { best = c; chosen[k][0] = a; chosen[k][1] = b; }
+            }
+            put(0, chosen[k][0], 1);
+            put(1, chosen[k][1], 1);
+            pa[k].ij = (uint32_t)(4 * chosen[k][0]) | ((uint32_t)(4 * chosen[k][1]) << 16);
+        }
+}
+
 // Builds the single device block of one ligand (see LigandDev).
 int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_params* ep,
                  std::vector<char>& blob, LigandDev& hd) {
@@ -306,9 +343,11 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
     hd.off_tor_move = take(sizeof(float4) * (T ? T : 1));
     hd.off_tor_atoms = take(sizeof(int2) * (T ? T : 1));
     const int PP = padded_pairs(P, kPairPad);
-    hd.off_pair_a = take(sizeof(PairA) * (P ? PP : 1));
+    const bool one = N > 32, two = N <= kSlotCopyAtoms;   // numbers of slot copies that can occur
+    if (one) hd.off_pair_a[0] = take(sizeof(PairA) * (P ? PP : 1));
+    if (two) hd.off_pair_a[1] = take(sizeof(PairA) * (P ? PP : 1));
     hd.off_pair_b = take(sizeof(PairB) * (P ? PP : 1));
-    hd.off_pair_x = take(sizeof(uint32_t) * (P ? PP : 1));
+    hd.off_pair_x = take(sizeof(PairX) * (P ? PP : 1));
     hd.off_type_ds = take(sizeof(float2) * NT);
     hd.total_bytes = (uint32_t)off;
     blob.assign(off, 0);
@@ -348,9 +387,9 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
     });
     float2* tds = reinterpret_cast<float2*>(blob.data() + hd.off_type_ds);
     for (int t = 0; t < NT; ++t) tds[t] = make_float2(L->ds_s[t], L->ds_v[t]);
-    PairA* pra = reinterpret_cast<PairA*>(blob.data() + hd.off_pair_a);
+    PairA* pra = reinterpret_cast<PairA*>(blob.data() + hd.off_pair_a[one ? 0 : 1]);
     PairB* prb = reinterpret_cast<PairB*>(blob.data() + hd.off_pair_b);
-    uint32_t* prx = reinterpret_cast<uint32_t*>(blob.data() + hd.off_pair_x);
+    PairX* prx = reinterpret_cast<PairX*>(blob.data() + hd.off_pair_x);
     for (int q = 0; q < P; ++q) {
         const int p = order[q];
         PairA& ra = pra[q];
@@ -364,9 +403,9 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
         bool cgg0 = (r1 == 24 && r2 == 25) || (r1 == 25 && r2 == 24);   // ATYPE_CG_IDX / ATYPE_G0_IDX
         bool fast = (m == 12) && (n == 6 || n == 10);
         if (!fast) hd.any_general = 1;
-        ra.ij = (uint32_t)(4 * i) | ((uint32_t)(4 * j) << 16);
         ra.fn = (float)n;
-        prx[q] = m | (n << 8) | (cgg0 ? kPairCgG0 : 0u) | (fast ? kPairFast : 0u);
+        prx[q].flags = m | (n << 8) | (cgg0 ? kPairCgG0 : 0u) | (fast ? kPairFast : 0u);
+        prx[q].atoms = (uint32_t)i | ((uint32_t)j << 16);
         ra.ac = L->vw_ac[idx];
         ra.bd = L->vw_bd[idx];
         rb.reqm = L->reqm_ab[idx];
@@ -378,10 +417,16 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
     }
     for (int q = P; P && q < PP; ++q) {   // padding (kPairPad): a real pair's geometry, no terms
         const int p = (q - P) % P;
-        pra[q].ij = pra[p].ij;
         pra[q].fn = 6.0f;
         prb[q].reqm = prb[p].reqm;
-        prx[q] = 12u | (6u << 8) | kPairFast;
+        prx[q].flags = 12u | (6u << 8) | kPairFast;
+        prx[q].atoms = prx[p].atoms;
+    }
+    if (one && two) std::memcpy(blob.data() + hd.off_pair_a[1], pra, sizeof(PairA) * PP);
+    for (int copies = 1; P && copies <= 2; ++copies) {
+        if (!(copies == 1 ? one : two)) continue;
+        PairA* out = reinterpret_cast<PairA*>(blob.data() + hd.off_pair_a[copies - 1]);
+        for (int q = 0; q < PP; q += 32) spread_slots(copies, slot_stride(N), prx + q, out + q);
     }
     std::memcpy(blob.data(), &hd, sizeof(hd));
     return ADGPU_OK;
@@ -1198,7 +1243,8 @@ static int enqueue_generation(adgpu_job_t j, int k, const LigandSet* ls, const M
     adgpu_context* c = j->ctx;
     RunGroup& g = j->groups[k];
     const int slot = (int)(g.enq % kRing);
-    const LaunchArgs la = launch_args(c, *ls, *ms, g.stream, (int)j->groups.size(), j->team_hint);
+    LaunchArgs la = launch_args(c, *ls, *ms, g.stream, (int)j->groups.size(), j->team_hint);
+    la.crowded = j->sharers > 1;
     const SearchDev sd = slice_sd(j, g.r0, g.r1);
     JobBuffers b = slice(j, g.r0, g.r1, g.parity, k);
     const int m = ls_method_for(j, j->generation + g.enq);

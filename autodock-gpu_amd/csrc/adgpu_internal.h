@@ -20,7 +20,7 @@ constexpr int kGenes = ADGPU_GENOTYPE_STRIDE;
 // are kept in the form the pair loop uses (byte offsets into its coordinate
 // arrays, a float), so that it spends no instruction on unpacking them.
 struct __attribute__((aligned(16))) PairA {
-    uint32_t ij;      // 4 * atom1 | (4 * atom2) << 16
+    uint32_t ij;      // 4 * slot1 | (4 * slot2) << 16 (atom slots, below)
     float fn;         // exponent n of the attractive term
     float ac;         // VWpars_AC of the type pair
     float bd;         // VWpars_BD
@@ -31,8 +31,30 @@ struct __attribute__((aligned(16))) PairB {
     float dsol;       // (S1 + qasp|q1|) V2 + (S2 + qasp|q2|) V1
     float g;          // CG-G0 bond constant G: 50 for a CG-G0 pair, else 0
 };
-// PairX flags: m | n << 8 | (CG-G0 bond) << 16 | (12-6 / 12-10 form) << 17.
+// What only rare paths read of a pair, in a third array.
+struct PairX {
+    uint32_t flags;   // m | n << 8 | (CG-G0 bond) << 16 | (12-6 / 12-10 form) << 17
+    uint32_t atoms;   // atom1 | atom2 << 16, in the order of the caller's list
+};
 constexpr uint32_t kPairCgG0 = 1u << 16, kPairFast = 1u << 17;
+
+// Atom slots of a team's LDS arrays (coordinates, force accumulators).  Lanes
+// of a half-wavefront that add to one address take 2m - 1 cycles for m lanes
+// (up to two addresses in one bank are free), and the pairs of a step share
+// atoms, so small ligands keep two copies of every atom, slot_stride apart:
+// copy c of atom a is slot c * slot_stride + a.  Two copies up to 32 atoms,
+// and up to 64 in 64-lane teams; 32-lane teams of more atoms keep one, because
+// eight teams' second copies would cost a workgroup its place on the compute
+// unit.  PairA is stored for either number where both can occur.
+constexpr int kSlotCopyAtoms = 64;
+__host__ __device__ constexpr int slot_copies(int TW, int NC) { return TW == 64 ? (NC == 1 ? 2 : 1) : (TW * NC <= 32 ? 2 : 1); }
+__host__ __device__ constexpr int slot_stride(int atoms) { return (atoms + 31) / 32 * 32 + 16; }
+// Words of one slot array of a team of TW lanes with NC atoms each: room for
+// the largest ligand of the shape (so that the arrays lie at fixed offsets)
+// and a slot for what lanes without an atom write.
+__host__ __device__ constexpr int slot_array(int TW, int NC) {
+    return slot_copies(TW, NC) == 2 ? 2 * slot_stride(TW * NC) : TW * NC + 4;
+}
 
 // The pair arrays are padded to a multiple of the widest team, so that every
 // lane of every team takes part in every step of the pair loop.  A padding
@@ -54,11 +76,11 @@ struct LigandDev {
     uint32_t off_tor_unit;    // float4 [T]  unit vector
     uint32_t off_tor_move;    // float4 [T]  moving vector
     uint32_t off_tor_atoms;   // int2   [T]  bond atoms
-    uint32_t off_pair_a;      // PairA[P padded to kPairPad]
+    uint32_t off_pair_a[2];   // PairA[P padded to kPairPad] for one and for two slot copies
     uint32_t off_pair_b;      // PairB[P padded]
-    uint32_t off_pair_x;      // uint32 [P padded] flags (PairX)
+    uint32_t off_pair_x;      // PairX[P padded]
     uint32_t off_type_ds;     // float2 [num_atypes] (dspars_S, dspars_V) per ligand type (FP64 re-scoring)
-    uint32_t total_bytes, pad6;
+    uint32_t total_bytes;
 };
 
 struct GridDev {
@@ -145,6 +167,7 @@ struct LaunchArgs {
     int team_hint;               // 0 = automatic, 32 or 64 = team width
     int share;                   // concurrent launches sharing the device (run groups); persistent
                                  // local-search grids take 1/share of the resident capacity
+    bool crowded = false;        // launches of other requests (a server's slots) run beside this one
 };
 
 // Launchers (k_*.hip).

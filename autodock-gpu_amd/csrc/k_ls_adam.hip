@@ -93,7 +93,7 @@ hipError_t launch_ls_adam(const LaunchArgs& la, const SearchDev& sp, const JobBu
     const int n = sp.num_runs * sp.num_ls;
     Launch a{};
     a.L = la.lig_dev; a.G = la.grid; a.S = sp; a.B = b;
-    const Shape sh = choose_shape(*la.lig_host, la.team_hint, ls_group_threads());
+    const Shape sh = choose_ls_shape(la, n, ls_group_threads());
     const int per_group = sh.threads / sh.tw;
     hipError_t err = hipSuccess;
     ADGPU_DISPATCH(k_ls_adam, sh, la.grid.format, {

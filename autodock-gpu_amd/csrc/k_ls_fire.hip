@@ -164,7 +164,7 @@ hipError_t launch_ls_fire(const LaunchArgs& la, const SearchDev& sp, const JobBu
     });
     if (err != hipSuccess) return err;
     // the persistent loop, in workgroups of ls_group_threads()
-    const Shape shl = choose_shape(*la.lig_host, la.team_hint, ls_group_threads());
+    const Shape shl = choose_ls_shape(la, n, ls_group_threads());
     const int want_l = (n + shl.threads / shl.tw - 1) / (shl.threads / shl.tw);
     ADGPU_DISPATCH(k_ls_fire, shl, la.grid.format, {
         const int cap = persistent_cap(reinterpret_cast<const void*>(kfn), shl.lds, shl.threads, la.share);

@@ -159,7 +159,7 @@ hipError_t launch_ls_sw(const LaunchArgs& la, const SearchDev& sp, const JobBuff
     a.L = la.lig_dev; a.G = la.grid; a.S = sp; a.B = b;
     a.lig_scale = 1.0f / sqrtf((float)la.lig_host->num_atoms);
     a.gene_scale = 1.0f / sqrtf((float)la.lig_host->num_genes);
-    const Shape sh = choose_shape(*la.lig_host, la.team_hint, ls_group_threads());
+    const Shape sh = choose_ls_shape(la, n, ls_group_threads());
     const int per_group = sh.threads / sh.tw;
     hipError_t err = hipSuccess;
     ADGPU_DISPATCH(k_ls_sw, sh, la.grid.format, {

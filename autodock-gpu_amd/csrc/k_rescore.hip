@@ -50,9 +50,9 @@ __global__ __launch_bounds__(64) void k_rescore_f64(const LigandDev* L, GridDev 
     const uint2* am = reinterpret_cast<const uint2*>(gb + L->off_atom_mask);
     const float4* tu = reinterpret_cast<const float4*>(gb + L->off_tor_unit);
     const float4* tm = reinterpret_cast<const float4*>(gb + L->off_tor_move);
-    const PairA* pa = reinterpret_cast<const PairA*>(gb + L->off_pair_a);
+    const PairA* pa = reinterpret_cast<const PairA*>(gb + L->off_pair_a[L->num_atoms > 32 ? 0 : 1]);
     const PairB* pb = reinterpret_cast<const PairB*>(gb + L->off_pair_b);
-    const uint32_t* px = reinterpret_cast<const uint32_t*>(gb + L->off_pair_x);
+    const PairX* px = reinterpret_cast<const PairX*>(gb + L->off_pair_x);
     const float2* tds = reinterpret_cast<const float2*>(gb + L->off_type_ds);
     const float* g = geno + (size_t)pose * kGenes;
     const double d2r = (double)kDegToRad;
@@ -119,8 +119,8 @@ __global__ __launch_bounds__(64) void k_rescore_f64(const LigandDev* L, GridDev 
     for (int k = lane; k < P; k += 64) {   // pair terms, calcenergy.cl:397-536
         const PairA A = pa[k];
         const PairB B = pb[k];
-        const uint32_t flags = px[k];
-        const int i = (int)(A.ij & 0xffffu) >> 2, j = (int)(A.ij >> 18);
+        const uint32_t flags = px[k].flags, atoms = px[k].atoms;
+        const int i = (int)(atoms & 0xffffu), j = (int)(atoms >> 16);
         const double sx = cx[i] - cx[j], sy = cy[i] - cy[j], sz = cz[i] - cz[j];
         const double dist = sqrt(sx * sx + sy * sy + sz * sz) * spacing;
         double e = (flags & kPairCgG0) ? 50.0 * dist : 0.0;   // CG-G0 bond term

@@ -60,3 +60,33 @@ def test_padded_pairs(gpu_ctx, c1, width):
     finally:
         gpu_ctx.set_team_width(0)
         gpu_ctx.maps_release(mid)
+
+
+@pytest.mark.parametrize("atoms, torsions, width", [(54, 8, 64), (72, 10, 64)])
+def test_large_workgroups(gpu_ctx, atoms, torsions, width):
+    """Local searches in the workgroups that a launch of many searches takes
+    when 256-thread ones could not all hold the pair records: the searches of
+    a job of 40 runs end as in a job of the first 2 runs, which fit at once."""
+    case = helpers.synthetic_case(atoms, torsions, lig_seed=atoms, map_seed=4, npts=40)
+    mid = gpu_ctx.maps_upload(case.packed, case.size, case.maps.num_map_atypes, case.spacing)
+    lid = gpu_ctx.ligand_upload(case.tables, case.ep)
+    gpu_ctx.set_team_width(width)
+    try:
+        pop, got = 150, []
+        init = O.initial_population((5,), 40, pop, case.maps.size_angstr, case.spacing)
+        seeds = O.cmwc_uints((5,), 40 * pop * 64)
+        for nrun in (40, 2):
+            sp = adgpu.search_params(num_runs=nrun, pop_size=pop, ls="adam", spacing=case.spacing, max_iters=12)
+            job = gpu_ctx.job(mid, lid, sp, init[:nrun * pop], seeds[:nrun * pop * 64])
+            job.initpop()
+            job.generation()
+            got.append(job.download())
+            job.destroy()
+        n = 2 * pop
+        assert np.array_equal(got[0]["pop"][:n], got[1]["pop"])
+        assert np.array_equal(got[0]["ene"][:n], got[1]["ene"])
+        helpers.check_energies(case.orc, got[0]["pop"][::97], got[0]["ene"][::97], edge_share=0.2)
+    finally:
+        gpu_ctx.set_team_width(0)
+        gpu_ctx.ligand_release(lid)
+        gpu_ctx.maps_release(mid)
