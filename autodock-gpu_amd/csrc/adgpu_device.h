@@ -59,9 +59,10 @@ DEV void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int CTRL>
+// ZERO: lanes without a source read 0.
+template <int CTRL, bool ZERO = false>
 DEV float dpp(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, ZERO));
 }
 DEV float rdl(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
 DEV int rdl_i(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
@@ -92,6 +93,19 @@ struct Team {
             const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
             v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
         }
+        return v;
+    }
+    // The same sum, the same bits, in the lanes of the team's last row only:
+    // each row's last lane is broadcast to the next row, then the first half's
+    // to the second, one instruction each where the row swaps take three.
+    static constexpr int kTop = TW - 16;
+    DEV static float sum_top(float v) {
+        v += dpp<0xB1>(v);
+        v += dpp<0x4E>(v);
+        v += dpp<0x141>(v);
+        v += dpp<0x140>(v);
+        if constexpr (TW >= 32) v += dpp<0x142, true>(v);
+        if constexpr (TW == 64) v += dpp<0x143, true>(v);
         return v;
     }
     // Value of team lane k (k uniform).
@@ -233,12 +247,19 @@ DEV float4 load_pt<ADGPU_MAP_BF16>(const void* base, uint32_t idx) {
 // ---------------------------------------------------------------------------
 // LDS layout
 // ---------------------------------------------------------------------------
+// One rotatable bond in a team's LDS block: its rotation, then (once the
+// coordinates are made) its axis; its moving vector; the bond's first atom.
+struct TorRec {
+    float4 q;
+    float4 m;
+    float4 r0;
+};
+
 struct SharedView {           // staged once per workgroup
     const PairA* pa;          // LDS (or global when the pairs do not fit): record p of step k is
     const PairB* pb;          //   [k * pair_stride<TW, PL> + lane] of both
     const PairX* px;          // global (rarely read)
     const float4* tor_unit;
-    const float4* tor_move;
     const int2* tor_atoms;
 };
 
@@ -253,11 +274,9 @@ struct TeamView {             // private to one team
     int* fx;                  // [slot_array] int32 fixed-point pair forces
     int* fy;
     int* fz;
-    float4* tq;               // [T] torsion quaternions
-    float4* tax;              // [T] torsion axes (gradient)
-    float4* tref;             // [T] torsion reference atoms (gradient)
-    int* gi;                  // [T][4] torsion gene gradients (int fixed point), in
-                              //   four parts: lanes add to the part of their index mod 4
+    TorRec* tor;              // [T]
+    int* gi;                  // [6 + T][4] gene gradients (int fixed point), in four
+                              //   parts: lanes add to the part of their index mod 4
     float* pg;                // [12] genes 0..5, sin/cos of phi, theta, rot/2
 };
 
@@ -271,12 +290,12 @@ constexpr int pair_stride = PL ? 2 * TW : TW;
 
 __host__ __device__ inline size_t shared_bytes_for(int TW, int T, int P, bool pairs_in_lds) {
     size_t s = pairs_in_lds ? (size_t)padded_pairs(P, TW) * (sizeof(PairA) + sizeof(PairB)) : 0;
-    s += (size_t)T * (sizeof(float4) * 2 + sizeof(int2));
+    s += (size_t)T * (sizeof(float4) + sizeof(int2));
     return align16(s);
 }
 
 __host__ __device__ inline size_t team_bytes_for(int TW, int NC, int T) {
-    return 6 * (size_t)slot_array(TW, NC) * 4 + (size_t)T * 48 + (size_t)T * 16 + 48;
+    return 6 * (size_t)slot_array(TW, NC) * 4 + (size_t)T * sizeof(TorRec) + (size_t)(6 + T) * 16 + 48;
 }
 
 // LDS of one workgroup of `threads` threads (threads / TW teams).
@@ -311,13 +330,12 @@ DEV void stage(const LigandDev* L, char* lds, SharedView& sv, TeamView& tv) {
         sv.pb = gpb;
     }
     float4* tu = reinterpret_cast<float4*>(p);
-    float4* tm = tu + T;
-    int2* ta = reinterpret_cast<int2*>(tm + T);
+    int2* ta = reinterpret_cast<int2*>(tu + T);
     const float4* gtu = reinterpret_cast<const float4*>(gbase + L->off_tor_unit);
     const float4* gtm = reinterpret_cast<const float4*>(gbase + L->off_tor_move);
     const int2* gta = reinterpret_cast<const int2*>(gbase + L->off_tor_atoms);
-    for (int k = threadIdx.x; k < T; k += blockDim.x) { tu[k] = gtu[k]; tm[k] = gtm[k]; ta[k] = gta[k]; }
-    sv.tor_unit = tu; sv.tor_move = tm; sv.tor_atoms = ta;
+    for (int k = threadIdx.x; k < T; k += blockDim.x) { tu[k] = gtu[k]; ta[k] = gta[k]; }
+    sv.tor_unit = tu; sv.tor_atoms = ta;
     char* w = lds + shared_bytes_for(TW, T, P, PL) + (size_t)(threadIdx.x / TW) * team_bytes_for(TW, NC, T);
     constexpr int kArray = slot_array(TW, NC);
     tv.cx = reinterpret_cast<float*>(w);
@@ -327,12 +345,11 @@ DEV void stage(const LigandDev* L, char* lds, SharedView& sv, TeamView& tv) {
     tv.fy = tv.fx + kArray;
     tv.fz = tv.fy + kArray;
     w += 6 * (size_t)kArray * 4;
-    tv.tq = reinterpret_cast<float4*>(w);
-    tv.tax = tv.tq + T;
-    tv.tref = tv.tax + T;
-    w += (size_t)T * 48;
+    tv.tor = reinterpret_cast<TorRec*>(w);
+    for (int t = Team<TW>::lane(); t < T; t += TW) tv.tor[t].m = gtm[t];
+    w += (size_t)T * sizeof(TorRec);
     tv.gi = reinterpret_cast<int*>(w);
-    w += (size_t)T * 16;
+    w += (size_t)(6 + T) * 16;
     tv.pg = reinterpret_cast<float*>(w);
     __syncthreads();
 }
@@ -344,7 +361,7 @@ template <int TW, int NC>
 struct Atoms {
     float3 ref[NC];
     float q[NC];
-    uint32_t mlo[NC], mhi[NC];
+    uint32_t mlo[NC];         // rotatable bonds 0..31 that move the atom
     uint32_t mapoff[NC];      // map index * g3
     uint32_t slot[NC];        // byte offset of the atom's first copy in the slot arrays
     uint32_t copy;            // bytes from there to its second copy
@@ -371,7 +388,6 @@ struct Atoms {
             ref[k] = make_float3(r.x, r.y, r.z);
             q[k] = r.w;
             mlo[k] = valid[k] ? m.x : 0u;
-            mhi[k] = valid[k] ? m.y : 0u;
             mapoff[k] = valid[k] ? (uint32_t)inf.x * G.g3 : 0u;
             ign[k] = !valid[k] || inf.z != 0;
             lig[k] = valid[k] && a < L->true_ligand_atoms;
@@ -403,6 +419,19 @@ struct EvalCtx {
     Atoms<TW, NC> A;
     LigScalars ls;
 };
+
+// Calls f(t) for the rotatable bonds t that move atom chunk k of the lane, in
+// ascending order.  Bonds beyond the 32nd are rare: their bits are read from
+// the ligand block instead of keeping a register.
+template <int TW, int NC, class F>
+DEV void for_bonds(const LigandDev* L, int T, const Atoms<TW, NC>& A, int k, F&& f) {
+    for (uint32_t m = A.mlo[k]; m; m &= m - 1) f(__builtin_ctz(m));
+    if (__builtin_expect(T > 32, 0)) {
+        const uint2* am = reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(L) + L->off_atom_mask);
+        uint32_t m = A.valid[k] ? am[Team<TW>::lane() + TW * k].y : 0u;
+        for (; m; m &= m - 1) f(32 + __builtin_ctz(m));
+    }
+}
 
 // ---------------------------------------------------------------------------
 // Pose (calcenergy.cl:201-221): genes 0..5 and the sine/cosine of the
@@ -437,7 +466,7 @@ DEV void gene_trig(const LigScalars& ls, const SharedView& sv, const TeamView& t
                 tv.pg[7 + 2 * (g - 3)] = c;
             } else {
                 float4 u = sv.tor_unit[g - 6];
-                tv.tq[g - 6] = make_float4(s * u.x, s * u.y, s * u.z, c);
+                tv.tor[g - 6].q = make_float4(s * u.x, s * u.y, s * u.z, c);
             }
         }
     }
@@ -469,21 +498,17 @@ DEV Pose read_pose(const TeamView& tv, bool has_ligand) {
 // moving it in ascending index, then the general rotation (the per-atom order
 // gen_rotlist encodes, host/src/calcenergy.cpp:387-488).
 template <int TW, int NC>
-DEV void compute_coords(const SharedView& sv, const TeamView& tv, const Atoms<TW, NC>& A, const Pose& P,
-                        float3 (&c)[NC]) {
+DEV void compute_coords(const EvalCtx<TW, NC>& X, const Pose& P, float3 (&c)[NC]) {
+    const TeamView& tv = X.tv;
+    const Atoms<TW, NC>& A = X.A;
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
         float3 v = A.ref[k];
-        uint32_t lo = A.mlo[k], hi = A.mhi[k];
-        while (lo | hi) {
-            int t;
-            if (lo) { t = __builtin_ctz(lo); lo &= lo - 1; }
-            else { t = 32 + __builtin_ctz(hi); hi &= hi - 1; }
-            float4 q = tv.tq[t];
-            float4 m = sv.tor_move[t];
+        for_bonds<TW, NC>(X.L, X.ls.T, A, k, [&](int t) {
+            const float4 q = tv.tor[t].q, m = tv.tor[t].m;
             float3 r = qrot(make_float3(v.x - m.x, v.y - m.y, v.z - m.z), q);
             v = make_float3(r.x + m.x, r.y + m.y, r.z + m.z);
-        }
+        });
         if (A.lig[k]) {
             float3 r = qrot(v, P.q);
             v = make_float3(r.x + P.mv.x, r.y + P.mv.y, r.z + P.mv.z);
@@ -650,12 +675,16 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
                 const uint32_t o = X.A.slot[k] + copy * X.A.copy;
                 *at(tv.fx, o) = 0; *at(tv.fy, o) = 0; *at(tv.fz, o) = 0;
             }
-        for (int t = tl; t < T; t += TW) reinterpret_cast<int4*>(tv.gi)[t] = make_int4(0, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < TM::kGPL; ++j) {
+            if (j > 0 && NG <= TW) break;
+            if (tl + TW * j < NG) reinterpret_cast<int4*>(tv.gi)[tl + TW * j] = make_int4(0, 0, 0, 0);
+        }
     }
     wave_sync();
     const Pose pose = read_pose(tv, has_lig);
     float3 c[NC];
-    compute_coords<TW, NC>(sv, tv, X.A, pose, c);
+    compute_coords<TW, NC>(X, pose, c);
 
     // with one atom per lane the map loads go out before the pair loop and
     // land while it runs; with more, each chunk is gathered after it (the
@@ -764,36 +793,36 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
             }
         }
     }
-    sfx = TM::sum(sfx); sfy = TM::sum(sfy); sfz = TM::sum(sfz);
-    tx = TM::sum(tx); ty = TM::sum(ty); tz = TM::sum(tz);
-    int ig = 0;
-    if (has_lig && tl < 6) {
+    // Rigid-body genes in lanes 0..5 of the team's last row, which the sums
+    // above reach: every lane runs one chain, its gene's operands selected, and
+    // one rounding to the fixed point.
+    sfx = TM::sum_top(sfx); sfy = TM::sum_top(sfy); sfz = TM::sum_top(sfz);
+    tx = TM::sum_top(tx); ty = TM::sum_top(ty); tz = TM::sum_top(tz);
+    if (has_lig) {
+#pragma clang fp contract(off)
+        const int r = tl - TM::kTop;
         // translation genes, calcMergedEneGra.cl:679-697
-        const int it0 = quant(kTermScale * sfx * spacing), it1 = quant(kTermScale * sfy * spacing),
-                  it2 = quant(kTermScale * sfz * spacing);
-        // rotation genes, calcMergedEneGra.cl:756-861
-        const float tl2 = tx * tx + ty * ty + tz * tz;
-        const float tlen = fast_sqrt(tl2);
+        const float move = kTermScale * (r == 0 ? sfx : r == 1 ? sfy : sfz) * spacing;
+        // rotation genes (3 phi, 4 theta, 5 angle), calcMergedEneGra.cl:756-861
+        const bool is_phi = r == 3, is_theta = r == 4, is_rot = r == 5;
+        const float tlen = fast_sqrt(fmaf(tz, tz, fmaf(tx, tx, ty * ty)));
+        const float tlen2 = tlen * tlen;
         const bool small = tlen < 1e-3f;
         const float oscale = small ? 1.0f : tlen * (1.0f / 1e-3f);
-        const float sc = small ? 0.5f - tlen * tlen * (1.0f / 48.0f) : 0.0005f * fast_rcp(tlen);
-        const float4 qt = make_float4(tx * sc, ty * sc, tz * sc, small ? 1.0f - tlen * tlen * 0.125f : 0.99999988f);
+        const float sc = small ? fmaf(tlen2, -1.0f / 48.0f, 0.5f) : 0.0005f * fast_rcp(tlen);
+        const float4 qt = make_float4(tx * sc, ty * sc, tz * sc, small ? fmaf(tlen2, -0.125f, 1.0f) : 0.99999988f);
         const float4 tq = qmul(qt, pose.q);
-        const float cur_phi = fmod_pi2(kTwoPi + pose.phi);
-        const float cur_theta = fmod_pi2(kTwoPi + pose.theta);
-        const float cur_rot = fmod_pi2(kTwoPi + pose.rotangle);
-        const float tgt_rot = 2.0f * fast_acos(tq.w);
-        const float inv_sin = fast_rsq(1.0f - tq.w * tq.w);
-        const float tgt_theta = kTwoPi + pose.is_theta_gt_pi * fast_acos(tq.z * inv_sin);
-        const float tgt_phi = fmod_pi2(atan2f(pose.is_theta_gt_pi * tq.y, pose.is_theta_gt_pi * tq.x) + kTwoPi);
-        const float gphi = oscale * (fmod_pi2(tgt_phi - cur_phi + kPi) - kPi);
-        const float gtheta = oscale * (fmod_pi2(tgt_theta - cur_theta + kPi) - kPi);
-        const float grot = oscale * (fmod_pi2(tgt_rot - cur_rot + kPi) - kPi);
+        const float inv_sin = fast_rsq(fmaf(-tq.w, tq.w, 1.0f));
+        const float ac = fast_acos(is_theta ? tq.z * inv_sin : tq.w);
+        const float at = atan2f(pose.is_theta_gt_pi * tq.y, pose.is_theta_gt_pi * tq.x);
+        const float target = is_phi ? fmod_pi2(at + kTwoPi) : is_theta ? fmaf(pose.is_theta_gt_pi, ac, kTwoPi) : 2.0f * ac;
+        const float current = fmod_pi2(fmaf(tv.pg[tl & 7], kDegToRad, kTwoPi));
+        const float turn = oscale * (fmod_pi2(target - current + kPi) - kPi);
         const float corr = 4.0f * pose.sin_half * pose.sin_half;
-        const int ir0 = quant(kTermScale * gphi * pose.sin_theta * pose.sin_theta * corr * kDegToRad);
-        const int ir1 = quant(kTermScale * gtheta * corr * kDegToRad);
-        const int ir2 = quant(kTermScale * grot * kDegToRad);
-        ig = tl == 0 ? it0 : tl == 1 ? it1 : tl == 2 ? it2 : tl == 3 ? ir0 : tl == 4 ? ir1 : ir2;
+        const float s = is_phi ? pose.sin_theta : 1.0f;
+        const float rot = kTermScale * turn * s * s * (is_rot ? 1.0f : corr) * kDegToRad;
+        const int ig = quant(r < 3 ? move : rot);
+        if ((unsigned)r < 6u) tv.gi[4 * r] = ig;
     }
     // torsion genes, calcMergedEneGra.cl:866-915
     for (int t = tl; t < T; t += TW) {
@@ -801,24 +830,20 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
         const float4 r0 = make_float4(tv.cx[ab.x], tv.cy[ab.x], tv.cz[ab.x], 0.f);
         const float ax = tv.cx[ab.y] - r0.x, ay = tv.cy[ab.y] - r0.y, az = tv.cz[ab.y] - r0.z;
         const float inv = fast_rsq(ax * ax + ay * ay + az * az);
-        tv.tax[t] = make_float4(ax * inv, ay * inv, az * inv, 0.f);
-        tv.tref[t] = r0;
+        tv.tor[t].q = make_float4(ax * inv, ay * inv, az * inv, 0.f);
+        tv.tor[t].r0 = r0;
     }
     wave_sync();
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-        uint32_t lo = X.A.mlo[k], hi = X.A.mhi[k];
-        while (lo | hi) {
-            int t;
-            if (lo) { t = __builtin_ctz(lo); lo &= lo - 1; }
-            else { t = 32 + __builtin_ctz(hi); hi &= hi - 1; }
-            const float4 ax = tv.tax[t], r0 = tv.tref[t];
+        for_bonds<TW, NC>(X.L, T, X.A, k, [&](int t) {
+            const float4 ax = tv.tor[t].q, r0 = tv.tor[t].r0;
             const float rx = c[k].x - r0.x, ry = c[k].y - r0.y, rz = c[k].z - r0.z;
             const float qx = ry * F[k].z - rz * F[k].y, qy = rz * F[k].x - rx * F[k].z,
                         qz = rx * F[k].y - ry * F[k].x;
             const float toa = (ax.x * qx + ax.y * qy + ax.z * qz) * spacing;
-            atomicAdd(&tv.gi[4 * t + (tl & 3)], quant(kTermScale * toa * kDegToRad));
-        }
+            atomicAdd(&tv.gi[24 + 4 * t + (tl & 3)], quant(kTermScale * toa * kDegToRad));
+        });
     }
     wave_sync();
     const float conv = spacing * spacing * 1.0f / (kDegToRad * kDegToRad);   // CONVERT_INTO_ANGSTROM_RADIAN
@@ -826,9 +851,8 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
     for (int j = 0; j < TM::kGPL; ++j) {
         const int g = tl + TW * j;
         int iv = 0;
-        if (g < 6) iv = ig;
-        else if (g < NG) {
-            const int4 part = reinterpret_cast<const int4*>(tv.gi)[g - 6];
+        if (g < NG) {
+            const int4 part = reinterpret_cast<const int4*>(tv.gi)[g];
             iv = part.x + part.y + part.z + part.w;
         }
         float gv = kOneOverTermScale * (float)iv;
@@ -869,7 +893,7 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
     wave_sync();
     const Pose pose = read_pose(tv, has_lig);
     float3 c[NC];
-    compute_coords<TW, NC>(sv, tv, X.A, pose, c);
+    compute_coords<TW, NC>(X, pose, c);
     wave_sync();
     float3 gin[NC];
     const uint32_t g3 = G.g3, ne = (uint32_t)(G.nmaps - 2) * g3, nd = ne + g3;
@@ -991,22 +1015,18 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
         const float4 r0 = make_float4(tv.cx[ab.x], tv.cy[ab.x], tv.cz[ab.x], 0.f);
         const float ax = tv.cx[ab.y] - r0.x, ay = tv.cy[ab.y] - r0.y, az = tv.cz[ab.y] - r0.z;
         const float inv = rsqrtf(ax * ax + ay * ay + az * az);
-        tv.tax[t] = make_float4(ax * inv, ay * inv, az * inv, 0.f);
-        tv.tref[t] = r0;
+        tv.tor[t].q = make_float4(ax * inv, ay * inv, az * inv, 0.f);
+        tv.tor[t].r0 = r0;
     }
     wave_sync();
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-        uint32_t lo = X.A.mlo[k], hi = X.A.mhi[k];
-        while (lo | hi) {
-            int t;
-            if (lo) { t = __builtin_ctz(lo); lo &= lo - 1; }
-            else { t = 32 + __builtin_ctz(hi); hi &= hi - 1; }
-            const float4 ax = tv.tax[t], r0 = tv.tref[t];
+        for_bonds<TW, NC>(X.L, T, X.A, k, [&](int t) {
+            const float4 ax = tv.tor[t].q, r0 = tv.tor[t].r0;
             const float rx = (c[k].x - r0.x) * spacing, ry = (c[k].y - r0.y) * spacing, rz = (c[k].z - r0.z) * spacing;
             const float qx = ry * F[k].z - rz * F[k].y, qy = rz * F[k].x - rx * F[k].z, qz = rx * F[k].y - ry * F[k].x;
             atomicAdd(&tacc[t], (ax.x * qx + ax.y * qy + ax.z * qz) * kDegToRad);
-        }
+        });
     }
     wave_sync();
     const float conv = spacing * spacing * 1.0f / (kDegToRad * kDegToRad);
