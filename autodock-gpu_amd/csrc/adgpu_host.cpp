@@ -127,6 +127,7 @@ struct adgpu_job {
     int32_t* evals_runs = nullptr;
     uint32_t* prng = nullptr;
     int32_t* counters = nullptr;        // one LS work-queue counter per group (16 ints apart)
+    float2* adam_pow = nullptr;         // ADAM's bias corrections (kAdamPow entries)
     int32_t* ls_ent = nullptr;
     float* ls_grad = nullptr;
     float* ls_state = nullptr;          // ADADELTA hand-off: saved searches, ring (cap_yield LS slots)
@@ -817,6 +818,7 @@ static int job_set_groups(adgpu_job* j, int ng, int nrun) {
 // Allocations of a job that do not depend on the request's size.
 static int job_open(adgpu_job* j) {
     bool ok = hipMalloc(&j->counters, 16 * kMaxGroups * sizeof(int32_t)) == hipSuccess &&
+              hipMalloc(&j->adam_pow, kAdamPow * sizeof(float2)) == hipSuccess &&
               hipMalloc(&j->d_stop, 16 * sizeof(int32_t)) == hipSuccess &&
               hipHostMalloc(&j->h_stop, 16 * sizeof(int32_t)) == hipSuccess &&
               hipEventCreateWithFlags(&j->ev_test, g_wait_event_flags.load()) == hipSuccess &&
@@ -954,6 +956,7 @@ static int job_start(adgpu_job* j, const adgpu_search_params* sp, const LigandDe
     HIPCHK(c, hipMemsetAsync(j->ene[1], 0, ne * sizeof(float), s));
     HIPCHK(c, hipMemsetAsync(j->counters, 0, 16 * kMaxGroups * sizeof(int32_t), s));
     HIPCHK(c, hipMemsetAsync(j->d_stop, 0, 16 * sizeof(int32_t), s));
+    if (sp->ls_method == ADGPU_LS_ADAM) HIPCHK(c, launch_adam_pow(s, j->sd, j->adam_pow));
     HIPCHK(c, hipStreamSynchronize(s));
     j->h_stop[0] = 0;
     return ADGPU_OK;
@@ -1027,7 +1030,7 @@ int adgpu_job_destroy(adgpu_job_t j) {
     (void)hipFree(j->ene[0]); (void)hipFree(j->ene[1]);
     (void)hipFree(j->evals_new); (void)hipFree(j->evals_runs); (void)hipFree(j->prng);
     (void)hipFree(j->d_ring);
-    (void)hipFree(j->counters); (void)hipFree(j->ls_ent); (void)hipFree(j->ls_grad);
+    (void)hipFree(j->counters); (void)hipFree(j->adam_pow); (void)hipFree(j->ls_ent); (void)hipFree(j->ls_grad);
     (void)hipFree(j->ls_state); (void)hipFree(j->ls_ring);
     (void)hipFree(j->d_stop); (void)hipFree(j->d_as); (void)hipFree(j->d_as_bins);
     (void)hipFree(j->d_as_log); (void)hipFree(j->d_as_out);
@@ -1076,6 +1079,7 @@ static JobBuffers slice(const adgpu_job* j, int r0, int r1, int parity, int coun
     b.ls_grad = j->ls_grad ? j->ls_grad + (size_t)r0 * nls * kGenes : nullptr;
     b.ls_state = j->ls_state ? j->ls_state + (size_t)r0 * nls * kAdStateFloats : nullptr;
     b.ls_ring = j->ls_ring ? j->ls_ring + 3 * (size_t)r0 * nls : nullptr;   // ring, then seats
+    b.adam_pow = j->adam_pow;
     b.stop = j->d_stop;
     (void)r1;
     return b;

@@ -118,6 +118,7 @@ inline int team_lanes_for(int n_atoms, int hint) {
 }
 
 constexpr int kAdStateFloats = 4 * kGenes + 8;
+constexpr int kAdamPow = 1024;   // entries of a job's table of ADAM's bias corrections
 
 struct JobBuffers {
     float* pop_cur;
@@ -136,6 +137,7 @@ struct JobBuffers {
     float* ls_state;       // ADADELTA hand-off: saved search per LS slot [runs*num_ls*kAdStateFloats]
     int32_t* ls_ring;      // ADADELTA hand-off: per claim of the queue, the search handed off there
                            // [runs*num_ls], then the regrouping seats [2*runs*num_ls]
+    const float2* adam_pow; // ADAM: (1 - beta1^t, 1 - beta2^t) for t = 1 .. kAdamPow
     const int32_t* stop;   // set by a passed AutoStop test: generation kernels return at once
     int32_t* evals_copy;   // when set, K2 also writes the new per-run totals here (a generation
                            // inside a captured graph block: its ring slot of the device copy)
@@ -185,6 +187,8 @@ hipError_t launch_ls_sw(const LaunchArgs& la, const SearchDev& sp, const JobBuff
 hipError_t launch_ls_ad(const LaunchArgs& la, const SearchDev& sp, const JobBuffers& b);
 hipError_t launch_ls_adam(const LaunchArgs& la, const SearchDev& sp, const JobBuffers& b);
 hipError_t launch_ls_fire(const LaunchArgs& la, const SearchDev& sp, const JobBuffers& b);
+// Fills a job's table of ADAM's bias corrections (kAdamPow entries).
+hipError_t launch_adam_pow(hipStream_t s, const SearchDev& sp, float2* table);
 // One AutoStop test (mode 0) or the final statistics (mode 1) on the
 // energies ene[num_runs*pop_size]; k_autostop.hip.
 hipError_t launch_autostop(hipStream_t s, const AutoStopParams& p, const float* ene, const int32_t* evals_runs,

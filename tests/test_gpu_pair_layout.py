@@ -90,3 +90,31 @@ def test_large_workgroups(gpu_ctx, atoms, torsions, width):
         gpu_ctx.set_team_width(0)
         gpu_ctx.ligand_release(lid)
         gpu_ctx.maps_release(mid)
+
+
+def test_adam_past_its_table(gpu_ctx, c1):
+    """ADAM searches around the end of the job's table of bias corrections
+    (1024 steps): a longer search keeps the shorter one's steps, so its best
+    energy is at most the shorter one's, and is the energy of its pose."""
+    mid = gpu_ctx.maps_upload(c1.packed, c1.size, c1.maps.num_map_atypes, c1.spacing)
+    lid = gpu_ctx.ligand_upload(c1.tables, c1.ep)
+    init = O.initial_population((9,), 1, 16, c1.maps.size_angstr, c1.spacing)
+    seeds = O.cmwc_uints((9,), 16 * 64)
+    last = None
+    for iters in (1023, 1024, 1025, 1100):
+        sp = adgpu.search_params(num_runs=1, pop_size=16, ls="adam", spacing=c1.spacing, max_iters=iters)
+        job = gpu_ctx.job(mid, lid, sp, init, seeds)
+        job.initpop()
+        job.kernel_gen()
+        job.kernel_ls()
+        job.sum_and_swap()
+        d = job.download()
+        job.destroy()
+        # the initial energies, 15 offspring, then one evaluation a step of every searched entity
+        assert int(d["evals_runs"][0]) == 16 + 15 + 16 * iters
+        helpers.check_energies(c1.orc, d["pop"], d["ene"], edge_share=0.3)
+        if last is not None:
+            assert np.all(d["ene"] <= last)
+        last = d["ene"]
+    gpu_ctx.ligand_release(lid)
+    gpu_ctx.maps_release(mid)
