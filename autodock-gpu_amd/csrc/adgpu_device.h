@@ -223,25 +223,33 @@ DEV float randf(uint32_t& s) {
 // ---------------------------------------------------------------------------
 // map gathers: one grid point of one map = 4 values (packed-4 layout)
 // ---------------------------------------------------------------------------
+// Bytes of a point, as a shift.
 template <int MF>
-DEV float4 load_pt(const void* base, uint32_t idx);
+constexpr int kPointShift = MF == ADGPU_MAP_F32 ? 4 : 3;
+
+template <int MF>
+DEV float4 load_pt(const void* p);
 
 template <>
-DEV float4 load_pt<ADGPU_MAP_F32>(const void* base, uint32_t idx) {
-    return reinterpret_cast<const float4*>(base)[idx];
+DEV float4 load_pt<ADGPU_MAP_F32>(const void* p) {
+    return *reinterpret_cast<const float4*>(p);
 }
 template <>
-DEV float4 load_pt<ADGPU_MAP_F16>(const void* base, uint32_t idx) {
-    uint2 r = reinterpret_cast<const uint2*>(base)[idx];
+DEV float4 load_pt<ADGPU_MAP_F16>(const void* p) {
+    uint2 r = *reinterpret_cast<const uint2*>(p);
     __half2 lo = *reinterpret_cast<__half2*>(&r.x), hi = *reinterpret_cast<__half2*>(&r.y);
     float2 a = __half22float2(lo), b = __half22float2(hi);
     return make_float4(a.x, a.y, b.x, b.y);
 }
 template <>
-DEV float4 load_pt<ADGPU_MAP_BF16>(const void* base, uint32_t idx) {
-    uint2 r = reinterpret_cast<const uint2*>(base)[idx];
+DEV float4 load_pt<ADGPU_MAP_BF16>(const void* p) {
+    uint2 r = *reinterpret_cast<const uint2*>(p);
     return make_float4(__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u),
                        __uint_as_float(r.y << 16), __uint_as_float(r.y & 0xffff0000u));
+}
+template <int MF>
+DEV float4 load_pt(const void* base, uint32_t idx) {
+    return load_pt<MF>(reinterpret_cast<const char*>(base) + ((uint64_t)idx << kPointShift<MF>));
 }
 
 // ---------------------------------------------------------------------------
@@ -539,12 +547,21 @@ DEV void gather_issue(const GridDev& G, float3 c, uint32_t mapoff, Gather<MF>& g
     // so no map index is ever formed from them
     g.in = (c.x >= 0.f) && (c.y >= 0.f) && (c.z >= 0.f) && (c.x < (float)(G.gx - 1)) &&
            (c.y < (float)(G.gy - 1)) && (c.z < (float)(G.gz - 1));
-    uint32_t p = 0;
-    if (g.in) p = (uint32_t)floorf(c.x) + (uint32_t)floorf(c.y) * G.g1 + (uint32_t)floorf(c.z) * G.g2;
-    const uint32_t ne = (uint32_t)(G.nmaps - 2) * G.g3, nd = ne + G.g3;
-    g.a0 = load_pt<MF>(G.data, mapoff + p); g.a1 = load_pt<MF>(G.data, mapoff + p + 1);
-    g.e0 = load_pt<MF>(G.data, ne + p); g.e1 = load_pt<MF>(G.data, ne + p + 1);
-    g.d0 = load_pt<MF>(G.data, nd + p); g.d1 = load_pt<MF>(G.data, nd + p + 1);
+    // Cell of the low corner; coordinates in the grid are not negative, so the
+    // conversion's truncation is their floor.  The e and d maps lie at uniform
+    // addresses, one 32-bit offset apart from which the loads reach both
+    // corners along x; only the type map's address is 64-bit arithmetic.
+    const uint32_t cell = (uint32_t)c.x + __umul24((uint32_t)c.y, G.g1) + __umul24((uint32_t)c.z, G.g2);
+    const uint32_t p = g.in ? cell : 0u;
+    constexpr uint32_t kPt = 1u << kPointShift<MF>;
+    const char* base = reinterpret_cast<const char*>(G.data);
+    const char* em = base + ((uint64_t)((uint32_t)(G.nmaps - 2) * G.g3) << kPointShift<MF>);
+    const char* dm = em + ((uint64_t)G.g3 << kPointShift<MF>);
+    const char* am = base + ((uint64_t)(mapoff + p) << kPointShift<MF>);
+    const uint32_t off = p << kPointShift<MF>;
+    g.a0 = load_pt<MF>(am); g.a1 = load_pt<MF>(am + kPt);
+    g.e0 = load_pt<MF>(em + off); g.e1 = load_pt<MF>(em + off + kPt);
+    g.d0 = load_pt<MF>(dm + off); g.d1 = load_pt<MF>(dm + off + kPt);
 }
 
 // The three maps are combined per cube corner first (type + q e + |q| d),
@@ -556,10 +573,9 @@ DEV float gather_finish(const GridDev& G, float3 c, float q, const Gather<MF>& g
         if (GRAD) { fi.x += 16777216; fi.y += 16777216; fi.z += 16777216; }
         return 16777216.0f;
     }
-    const float xl = floorf(c.x), yl = floorf(c.y), zl = floorf(c.z);
-    const float dx = c.x - xl, omdx = 1.0f - dx;
-    const float dy = c.y - yl, omdy = 1.0f - dy;
-    const float dz = c.z - zl, omdz = 1.0f - dz;
+    const float dx = __builtin_amdgcn_fractf(c.x), omdx = 1.0f - dx;
+    const float dy = __builtin_amdgcn_fractf(c.y), omdy = 1.0f - dy;
+    const float dz = __builtin_amdgcn_fractf(c.z), omdz = 1.0f - dz;
     const float aq = fabsf(q);
     // cube corner k: 0 000, 1 010, 2 001, 3 011 (low x: .x .y .z .w of a0/e0/d0), 4..7 the same at x+1
     const float4 l = make_float4(fmaf(aq, g.d0.x, fmaf(q, g.e0.x, g.a0.x)), fmaf(aq, g.d0.y, fmaf(q, g.e0.y, g.a0.y)),
