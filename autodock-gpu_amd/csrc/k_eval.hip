@@ -12,7 +12,7 @@ namespace adgpu {
 // nothing, so every wavefront runs the evaluation with all lanes.
 template <int TW, int NC, int MF, bool PL>
 __global__ ADGPU_GROUP_KERNEL void k_eval_poses(Launch a) {
-    KERNEL_PROLOGUE(TW, NC, PL)
+    KERNEL_PROLOGUE(TW, NC, PL, true)
     const bool live = team_idx < a.n;
     if (!TM::any_in_wave(live)) return;
     const int id = live ? team_idx : a.n - 1;
@@ -83,7 +83,7 @@ hipError_t eval_poses_noalloc(const LaunchArgs& la, float* scratch_dev, int mode
 }
 
 size_t lds_bytes(const LigandDev& Lh, int team_hint, int* team_width) {
-    Shape s = choose_shape(Lh, team_hint);
+    Shape s = choose_shape(Lh, team_hint, true);
     if (team_width) *team_width = s.tw;
     return s.lds;
 }
@@ -94,7 +94,7 @@ hipError_t launch_eval_poses(const LaunchArgs& la, int mode, const float* genoty
     Launch a{};
     a.L = la.lig_dev; a.G = la.grid; a.in_geno = genotypes; a.out_e = energies; a.out_g = grads; a.n = n;
     a.mode = mode;
-    const Shape sh = choose_shape(*la.lig_host, la.team_hint);
+    const Shape sh = choose_shape(*la.lig_host, la.team_hint, true);
     const int per_group = 256 / sh.tw;
     const dim3 grid((n + per_group - 1) / per_group);
     hipError_t err = hipSuccess;

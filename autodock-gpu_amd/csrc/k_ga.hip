@@ -11,7 +11,7 @@ namespace adgpu {
 // K1: energies of the initial population (kernel1.cl:28-145).
 template <int TW, int NC, int MF, bool PL>
 __global__ ADGPU_GROUP_KERNEL void k_initpop(Launch a) {
-    KERNEL_PROLOGUE(TW, NC, PL)
+    KERNEL_PROLOGUE(TW, NC, PL, false)
     const int ne = a.S.num_runs * a.S.pop_size;
     const bool live = team_idx < ne;
     if (!TM::any_in_wave(live)) return;
@@ -19,7 +19,7 @@ __global__ ADGPU_GROUP_KERNEL void k_initpop(Launch a) {
     float gene[GPL], grad[GPL];
 #pragma unroll
     for (int j = 0; j < GPL; ++j) gene[j] = a.B.pop_cur[(size_t)id * kGenes + tl + TW * j];
-    const float e = evaluate<TW, NC, MF, PL, false>(X, gene, grad);
+    const float e = evaluate<TW, NC, MF, PL, false, false>(X, gene, grad);
     if (live && tl == 0) { a.B.ene_cur[id] = e; a.B.evals_new[id] = 1; }
 }
 
@@ -30,7 +30,7 @@ __global__ ADGPU_GROUP_KERNEL void k_initpop(Launch a) {
 template <int TW, int NC, int MF, bool PL>
 __global__ ADGPU_GROUP_KERNEL void k_gen(Launch a) {
     if (JOB_STOPPED(a.B)) return;
-    KERNEL_PROLOGUE(TW, NC, PL)
+    KERNEL_PROLOGUE(TW, NC, PL, false)
     const int pop = a.S.pop_size, NG = a.S.num_genes;
     const int ne = a.S.num_runs * pop;
     const bool live = team_idx < ne;
@@ -42,7 +42,7 @@ __global__ ADGPU_GROUP_KERNEL void k_gen(Launch a) {
     k4_prepare<TW>(a.S, a.B.pop_cur + (size_t)run * pop * kGenes, a.B.ene_cur + (size_t)run * pop, st, ent, it);
     float in[GPL], grad[GPL];
     k4_genes<TW>(it, NG, in);
-    const float e = evaluate<TW, NC, MF, PL, false>(X, in, grad);
+    const float e = evaluate<TW, NC, MF, PL, false, false>(X, in, grad);
     if (!live) return;
     k4_store<TW>(it, NG, e, a.B.pop_next + (size_t)idx * kGenes, a.B.ene_next + idx, a.B.evals_new + idx, st);
 }
@@ -77,7 +77,7 @@ hipError_t launch_initpop(const LaunchArgs& la, const SearchDev& sp, const JobBu
     if (n <= 0) return hipSuccess;
     Launch a{};
     a.L = la.lig_dev; a.G = la.grid; a.S = sp; a.B = b;
-    const Shape sh = choose_shape(*la.lig_host, la.team_hint);
+    const Shape sh = choose_shape(*la.lig_host, la.team_hint, false);
     const int per_group = 256 / sh.tw;
     const dim3 grid((n + per_group - 1) / per_group);
     hipError_t err = hipSuccess;
@@ -93,7 +93,7 @@ hipError_t launch_gen(const LaunchArgs& la, const SearchDev& sp, const JobBuffer
     if (n <= 0) return hipSuccess;
     Launch a{};
     a.L = la.lig_dev; a.G = la.grid; a.S = sp; a.B = b;
-    const Shape sh = choose_shape(*la.lig_host, la.team_hint);
+    const Shape sh = choose_shape(*la.lig_host, la.team_hint, false);
     const int per_group = 256 / sh.tw;
     const dim3 grid((n + per_group - 1) / per_group);
     hipError_t err = hipSuccess;

@@ -119,7 +119,7 @@ DEV int seat_swap(int32_t* e, int v) {
 template <int TW, int NC, int MF, bool PL>
 __global__ ADGPU_GROUP_KERNEL void k_ls_ad(Launch a) {
     if (JOB_STOPPED(a.B)) return;
-    KERNEL_PROLOGUE(TW, NC, PL)
+    KERNEL_PROLOGUE(TW, NC, PL, true)
     const SearchDev& S = a.S;
     const int nls = S.num_ls, pop = S.pop_size, NG = S.num_genes;
     const int ntot = S.num_runs * nls;
@@ -333,7 +333,7 @@ hipError_t launch_ls_ad(const LaunchArgs& la, const SearchDev& sp, const JobBuff
     const int n = sp.num_runs * sp.num_ls;
     Launch a{};
     a.L = la.lig_dev; a.G = la.grid; a.S = sp; a.B = b;
-    const Shape sh = choose_ls_shape(la, n, ls_group_threads());
+    const Shape sh = choose_ls_shape(la, n, true, ls_group_threads());
     const int per_group = sh.threads / sh.tw;
     hipError_t err = hipSuccess;
     ADGPU_DISPATCH(k_ls_ad, sh, la.grid.format, {

@@ -26,7 +26,7 @@ __global__ __launch_bounds__(256) void k_adam_pow(float beta1, float beta2, floa
 template <int TW, int NC, int MF, bool PL>
 __global__ ADGPU_GROUP_KERNEL void k_ls_adam(Launch a) {
     if (JOB_STOPPED(a.B)) return;
-    KERNEL_PROLOGUE(TW, NC, PL)
+    KERNEL_PROLOGUE(TW, NC, PL, true)
     const SearchDev& S = a.S;
     const int nls = S.num_ls, pop = S.pop_size, NG = S.num_genes;
     const int ntot = S.num_runs * nls;
@@ -110,7 +110,7 @@ hipError_t launch_ls_adam(const LaunchArgs& la, const SearchDev& sp, const JobBu
     const int n = sp.num_runs * sp.num_ls;
     Launch a{};
     a.L = la.lig_dev; a.G = la.grid; a.S = sp; a.B = b;
-    const Shape sh = choose_ls_shape(la, n, ls_group_threads());
+    const Shape sh = choose_ls_shape(la, n, true, ls_group_threads());
     const int per_group = sh.threads / sh.tw;
     hipError_t err = hipSuccess;
     ADGPU_DISPATCH(k_ls_adam, sh, la.grid.format, {

@@ -14,7 +14,7 @@ namespace adgpu {
 template <int TW, int NC, int MF, bool PL>
 __global__ ADGPU_GROUP_KERNEL void k_fire_init(Launch a) {
     if (JOB_STOPPED(a.B)) return;
-    KERNEL_PROLOGUE(TW, NC, PL)
+    KERNEL_PROLOGUE(TW, NC, PL, true)
     const SearchDev& S = a.S;
     const int nls = S.num_ls, pop = S.pop_size, NG = S.num_genes;
     const int ntot = S.num_runs * nls;
@@ -47,7 +47,7 @@ __global__ ADGPU_GROUP_KERNEL void k_fire_init(Launch a) {
 template <int TW, int NC, int MF, bool PL>
 __global__ ADGPU_GROUP_KERNEL void k_ls_fire(Launch a) {
     if (JOB_STOPPED(a.B)) return;
-    KERNEL_PROLOGUE(TW, NC, PL)
+    KERNEL_PROLOGUE(TW, NC, PL, true)
     const SearchDev& S = a.S;
     const int nls = S.num_ls, pop = S.pop_size, NG = S.num_genes;
     const int ntot = S.num_runs * nls;
@@ -154,7 +154,7 @@ hipError_t launch_ls_fire(const LaunchArgs& la, const SearchDev& sp, const JobBu
     const int n = sp.num_runs * sp.num_ls;
     Launch a{};
     a.L = la.lig_dev; a.G = la.grid; a.S = sp; a.B = b;
-    const Shape sh = choose_shape(*la.lig_host, la.team_hint);
+    const Shape sh = choose_shape(*la.lig_host, la.team_hint, true);
     const int per_group = 256 / sh.tw;
     const int want = (n + per_group - 1) / per_group;
     hipError_t err = hipSuccess;
@@ -164,7 +164,7 @@ hipError_t launch_ls_fire(const LaunchArgs& la, const SearchDev& sp, const JobBu
     });
     if (err != hipSuccess) return err;
     // the persistent loop, in workgroups of ls_group_threads()
-    const Shape shl = choose_ls_shape(la, n, ls_group_threads());
+    const Shape shl = choose_ls_shape(la, n, true, ls_group_threads());
     const int want_l = (n + shl.threads / shl.tw - 1) / (shl.threads / shl.tw);
     ADGPU_DISPATCH(k_ls_fire, shl, la.grid.format, {
         const int cap = persistent_cap(reinterpret_cast<const void*>(kfn), shl.lds, shl.threads, la.share);

@@ -20,7 +20,7 @@ namespace adgpu {
 template <int TW, int NC, int MF, bool PL>
 __global__ ADGPU_GROUP_KERNEL void k_ls_sw(Launch a) {
     if (JOB_STOPPED(a.B)) return;
-    KERNEL_PROLOGUE(TW, NC, PL)
+    KERNEL_PROLOGUE(TW, NC, PL, false)
     const SearchDev& S = a.S;
     const int nls = S.num_ls, pop = S.pop_size, NG = S.num_genes;
     const int ntot = S.num_runs * nls;
@@ -99,7 +99,7 @@ __global__ ADGPU_GROUP_KERNEL void k_ls_sw(Launch a) {
             }
         }
         float grad[GPL];
-        const float ce = evaluate<TW, NC, MF, PL, false>(X, cand, grad);
+        const float ce = evaluate<TW, NC, MF, PL, false, false>(X, cand, grad);
         if (!done) {
             evals++;
             bool iter_end = false;
@@ -159,7 +159,7 @@ hipError_t launch_ls_sw(const LaunchArgs& la, const SearchDev& sp, const JobBuff
     a.L = la.lig_dev; a.G = la.grid; a.S = sp; a.B = b;
     a.lig_scale = 1.0f / sqrtf((float)la.lig_host->num_atoms);
     a.gene_scale = 1.0f / sqrtf((float)la.lig_host->num_genes);
-    const Shape sh = choose_ls_shape(la, n, ls_group_threads());
+    const Shape sh = choose_ls_shape(la, n, false, ls_group_threads());
     const int per_group = sh.threads / sh.tw;
     hipError_t err = hipSuccess;
     ADGPU_DISPATCH(k_ls_sw, sh, la.grid.format, {

@@ -62,8 +62,9 @@ def test_padded_pairs(gpu_ctx, c1, width):
         gpu_ctx.maps_release(mid)
 
 
-@pytest.mark.parametrize("atoms, torsions, width", [(54, 8, 64), (72, 10, 64)])
-def test_large_workgroups(gpu_ctx, atoms, torsions, width):
+@pytest.mark.parametrize("ls", ["adam", "sw"])
+@pytest.mark.parametrize("atoms, torsions, width", [(54, 8, 64), (72, 10, 64), (45, 8, 32)])
+def test_large_workgroups(gpu_ctx, atoms, torsions, width, ls):
     """Local searches in the workgroups that a launch of many searches takes
     when 256-thread ones could not all hold the pair records: the searches of
     a job of 40 runs end as in a job of the first 2 runs, which fit at once."""
@@ -76,7 +77,7 @@ def test_large_workgroups(gpu_ctx, atoms, torsions, width):
         init = O.initial_population((5,), 40, pop, case.maps.size_angstr, case.spacing)
         seeds = O.cmwc_uints((5,), 40 * pop * 64)
         for nrun in (40, 2):
-            sp = adgpu.search_params(num_runs=nrun, pop_size=pop, ls="adam", spacing=case.spacing, max_iters=12)
+            sp = adgpu.search_params(num_runs=nrun, pop_size=pop, ls=ls, spacing=case.spacing, max_iters=12)
             job = gpu_ctx.job(mid, lid, sp, init[:nrun * pop], seeds[:nrun * pop * 64])
             job.initpop()
             job.generation()
