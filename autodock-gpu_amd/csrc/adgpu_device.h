@@ -1199,7 +1199,7 @@ inline Shape choose_ls_shape(const LaunchArgs& la, int searches, bool grad, int 
     // wavefronts of all the launches that share the device, were they like this one
     const int64_t need = ((int64_t)searches * s.tw + kWave - 1) / kWave * la.share;
     int64_t best = INT64_MIN;
-    for (int t = kGroupThreads; t <= 1024; t += 128) {
+    for (int t = kGroupThreads; t <= 4 * kGroupThreads; t += kGroupThreads) {   // whole rounds of the four SIMDs
         const size_t lds = lds_bytes_for(s.tw, s.nc, L.num_rotbonds, L.num_pairs, true, grad, t);
         const int w = t / kWave, fit = groups_per_cu(lds, t);
         const int64_t groups = (need + w - 1) / w;
