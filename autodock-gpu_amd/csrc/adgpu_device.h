@@ -450,16 +450,44 @@ struct EvalCtx {
     LigScalars ls;
 };
 
-// Calls f(t) for the rotatable bonds t that move atom chunk k of the lane, in
-// ascending order.  Bonds beyond the 32nd are rare: their bits are read from
-// the ligand block instead of keeping a register.
+// Calls f(t, q, v) for the rotatable bonds t that move atom chunk k of the
+// lane, in ascending order, with the bond's record members `second` (v) and q.
+// 64-lane teams read the next bond's members while f runs, so that only the
+// first read's latency shows; 32-lane ones have no registers for it (ADAM, 41
+// atoms, 64 lanes 400 -> 452 M evals/s; ADADELTA, 30 atoms, 32 lanes 366 -> 371
+// ms a docking, were it done there).  Bonds beyond the 32nd are rare: their bits are read from the
+// ligand block instead of keeping a register.
 template <int TW, int NC, class F>
-DEV void for_bonds(const LigandDev* L, int T, const Atoms<TW, NC>& A, int k, F&& f) {
-    for (uint32_t m = A.mlo[k]; m; m &= m - 1) f(__builtin_ctz(m));
+DEV void for_bonds(const EvalCtx<TW, NC>& X, int k, float4 TorRec::*second, F&& f) {
+    const TorRec* tor = X.tv.tor;
+    const int T = X.ls.T;
+    if (uint32_t m = X.A.mlo[k]) {
+        int t = __builtin_ctz(m);
+        float4 q = tor[t].q, v = tor[t].*second;
+        for (;;) {
+            m &= m - 1;
+            if constexpr (TW == 64) {
+                const int next = m ? __builtin_ctz(m) : t;
+                const float4 nq = tor[next].q, nv = tor[next].*second;
+                f(t, q, v);
+                if (!m) break;
+                t = next; q = nq; v = nv;
+            } else {
+                f(t, q, v);
+                if (!m) break;
+                t = __builtin_ctz(m);
+                q = tor[t].q; v = tor[t].*second;
+            }
+        }
+    }
     if (__builtin_expect(T > 32, 0)) {
+        const LigandDev* L = X.L;
         const uint2* am = reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(L) + L->off_atom_mask);
-        uint32_t m = A.valid[k] ? am[Team<TW>::lane() + TW * k].y : 0u;
-        for (; m; m &= m - 1) f(32 + __builtin_ctz(m));
+        uint32_t m = X.A.valid[k] ? am[Team<TW>::lane() + TW * k].y : 0u;
+        for (; m; m &= m - 1) {
+            const int t = 32 + __builtin_ctz(m);
+            f(t, tor[t].q, tor[t].*second);
+        }
     }
 }
 
@@ -534,8 +562,7 @@ DEV void compute_coords(const EvalCtx<TW, NC>& X, const Pose& P, float3 (&c)[NC]
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
         float3 v = A.ref[k];
-        for_bonds<TW, NC>(X.L, X.ls.T, A, k, [&](int t) {
-            const float4 q = tv.tor[t].q, m = tv.tor[t].m;
+        for_bonds<TW, NC>(X, k, &TorRec::m, [&](int, const float4& q, const float4& m) {
             float3 r = qrot(make_float3(v.x - m.x, v.y - m.y, v.z - m.z), q);
             v = make_float3(r.x + m.x, r.y + m.y, r.z + m.z);
         });
@@ -876,8 +903,7 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
     wave_sync();
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-        for_bonds<TW, NC>(X.L, T, X.A, k, [&](int t) {
-            const float4 ax = tv.tor[t].q, r0 = tv.tor[t].r0;
+        for_bonds<TW, NC>(X, k, &TorRec::r0, [&](int t, const float4& ax, const float4& r0) {
             const float rx = c[k].x - r0.x, ry = c[k].y - r0.y, rz = c[k].z - r0.z;
             const float qx = ry * F[k].z - rz * F[k].y, qy = rz * F[k].x - rx * F[k].z,
                         qz = rx * F[k].y - ry * F[k].x;
@@ -1063,8 +1089,7 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
     wave_sync();
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-        for_bonds<TW, NC>(X.L, T, X.A, k, [&](int t) {
-            const float4 ax = tv.tor[t].q, r0 = tv.tor[t].r0;
+        for_bonds<TW, NC>(X, k, &TorRec::r0, [&](int t, const float4& ax, const float4& r0) {
             const float rx = (c[k].x - r0.x) * spacing, ry = (c[k].y - r0.y) * spacing, rz = (c[k].z - r0.z) * spacing;
             const float qx = ry * F[k].z - rz * F[k].y, qy = rz * F[k].x - rx * F[k].z, qz = rx * F[k].y - ry * F[k].x;
             atomicAdd(&tacc[t], (ax.x * qx + ax.y * qy + ax.z * qz) * kDegToRad);
