@@ -983,19 +983,28 @@ int adgpu_job_create(adgpu_ctx c, int map_id, int lig_id, const adgpu_search_par
     j->ligand_id = lig_id;
     const int nrun = sp->num_runs;
     // run groups: ADGPU_RUN_GROUPS streams.  Groups whose streams share a
-    // hardware queue serialize, so the default follows the HIP runtime's
-    // hardware queues per process (GPU_MAX_HW_QUEUES, 4 unless set): 2 groups
-    // (with the context's stream, 3 of 4 queues), or 4 groups when at least
-    // 6 queues are available (the faster setting on MI355X).  A group's
-    // local-search launch should still fill a good part of the device, so
-    // small jobs get fewer groups: one per kGroupSearches searches of a
-    // generation (measured: nrun 20 x 150 searches fastest in 2 groups,
-    // nrun 50 x 150 in 4)
-    int ng = 2;
+    // hardware queue serialize, so there are at most four, with the HIP
+    // runtime's four hardware queues per process (GPU_MAX_HW_QUEUES) or more,
+    // and two with fewer.  A group's local-search launch should still fill a
+    // good part of the device, so small jobs get fewer groups: one per
+    // kGroupSearches searches of a generation.  Launches in workgroups above
+    // 256 threads (large pair lists) overlap worse: two groups.  ms a docking
+    // in 1 / 2 / 3 / 4 groups on four queues: FIRE nrun 20, 30 atoms 49 / 47 /
+    // 52 / 59; Solis-Wets nrun 50, 30 atoms 72 / 59 / 60 / 58; ADADELTA nrun
+    // 100, 23 atoms 64 / 57 / 57 / 52, 30 atoms - / 364 / 369 / 346; ADAM nrun
+    // 50, 41 atoms - / 116 / 116 / 111; ADADELTA nrun 50, 54 atoms (512
+    // threads) - / 186 / 195 / 191.  Six groups on four queues: twice the time
+    // of two.
+    int ng = 4;
     if (const char* q = std::getenv("GPU_MAX_HW_QUEUES"))
-        if (std::atoi(q) >= 6) ng = 4;
+        if (std::atoi(q) >= 1 && std::atoi(q) < 4) ng = 2;
     const int64_t searches = (int64_t)nrun * std::max(1, to_dev(sp, num_genes).num_ls);
     ng = (int)std::max<int64_t>(1, std::min<int64_t>(ng, searches / kGroupSearches));
+    if (ng > 2) {
+        const int tw = job_team_width(c, li->second.host.num_atoms, searches, 1, sp->ls_method);
+        LaunchArgs la = launch_args(c, li->second, mi->second, nullptr, 1, tw);
+        if (ls_workgroup(la, (int)std::min<int64_t>(searches, INT32_MAX), sp->ls_method) > kGroupThreads) ng = 2;
+    }
     if (const char* e = std::getenv("ADGPU_RUN_GROUPS")) ng = std::atoi(e);
     rc = job_open(j.get());
     if (!rc) rc = job_set_groups(j.get(), ng, nrun);

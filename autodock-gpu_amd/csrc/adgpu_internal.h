@@ -204,6 +204,8 @@ hipError_t eval_poses_noalloc(const LaunchArgs& la, float* scratch_dev, int mode
 // FMA chains over `blocks` workgroups of 256 threads (k_calib.hip); scratch
 // holds blocks * 256 floats.
 hipError_t measure_valu_rate(hipStream_t stream, float* scratch, int blocks, int iters, double* wave_instr_per_s);
+// Threads of the workgroups that a local-search launch of so many searches takes.
+int ls_workgroup(const LaunchArgs& la, int searches, int method);
 // LDS bytes and team width the launchers use for a ligand.
 size_t lds_bytes(const LigandDev& lig_host, int team_hint, int* team_width);
 

@@ -109,6 +109,10 @@ hipError_t launch_sum_evals(hipStream_t s, const SearchDev& sp, const JobBuffers
     return hipGetLastError();
 }
 
+int ls_workgroup(const LaunchArgs& la, int searches, int method) {
+    return choose_ls_shape(la, searches, method != ADGPU_LS_SW, ls_group_threads()).threads;
+}
+
 hipError_t launch_ls(const LaunchArgs& la, const SearchDev& sp, const JobBuffers& b, int method) {
     if (sp.num_runs * sp.num_ls <= 0 || method == ADGPU_LS_NONE) return hipSuccess;
     const int n = sp.num_runs * sp.num_ls;
