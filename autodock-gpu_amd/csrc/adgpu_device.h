@@ -1117,6 +1117,7 @@ struct Launch {
     SearchDev S;
     JobBuffers B;
     const float* in_geno;
+    int stride;          // floats from one genotype (and gradient) to the next
     float* out_e;
     float* out_g;
     int n;

@@ -174,9 +174,11 @@ struct LaunchArgs {
 
 // Launchers (k_*.hip).
 // FP64 energies of n poses (k_rescore.hip): total, inter and intra per pose.
-hipError_t launch_rescore_f64(const LaunchArgs& la, const float* genotypes, int n, double* out3);
-hipError_t launch_eval_poses(const LaunchArgs& la, int mode, const float* genotypes, int n, float* energies,
-                             float* grads);
+// stride: floats from one genotype to the next (at least the ligand's genes).
+hipError_t launch_rescore_f64(const LaunchArgs& la, const float* genotypes, int stride, int n, double* out3);
+// Energies and gradients of n poses; gradients lie `stride` floats apart too.
+hipError_t launch_eval_poses(const LaunchArgs& la, int mode, const float* genotypes, int stride, int n,
+                             float* energies, float* grads);
 hipError_t launch_initpop(const LaunchArgs& la, const SearchDev& sp, const JobBuffers& b);
 hipError_t launch_gen(const LaunchArgs& la, const SearchDev& sp, const JobBuffers& b);
 hipError_t launch_sum_evals(hipStream_t s, const SearchDev& sp, const JobBuffers& b);

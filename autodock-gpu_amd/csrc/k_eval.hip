@@ -18,7 +18,7 @@ __global__ ADGPU_GROUP_KERNEL void k_eval_poses(Launch a) {
     const int id = live ? team_idx : a.n - 1;
     float gene[GPL], grad[GPL];
 #pragma unroll
-    for (int j = 0; j < GPL; ++j) gene[j] = a.in_geno[(size_t)id * kGenes + tl + TW * j];
+    for (int j = 0; j < GPL; ++j) gene[j] = tl + TW * j < a.stride ? a.in_geno[(size_t)id * a.stride + tl + TW * j] : 0.f;
     if (a.mode == ADGPU_EVAL_GRADIENT) {
         float_gradient<TW, NC, MF, PL>(X, gene, grad);
     } else if (a.mode == ADGPU_EVAL_ENERGRAD) {
@@ -31,7 +31,8 @@ __global__ ADGPU_GROUP_KERNEL void k_eval_poses(Launch a) {
     }
     if (live && a.out_g) {
 #pragma unroll
-        for (int j = 0; j < GPL; ++j) a.out_g[(size_t)id * kGenes + tl + TW * j] = grad[j];
+        for (int j = 0; j < GPL; ++j)
+            if (tl + TW * j < a.stride) a.out_g[(size_t)id * a.stride + tl + TW * j] = grad[j];
     }
 }
 
@@ -73,7 +74,7 @@ hipError_t eval_poses_noalloc(const LaunchArgs& la, float* scratch_dev, int mode
     float* d_ene = scratch_dev + 2 * cap * kGenes;
     hipError_t e = hipMemcpyAsync(d_geno, genotypes, sizeof(float) * kGenes * (size_t)n, hipMemcpyHostToDevice,
                                   la.stream);
-    if (e == hipSuccess) e = launch_eval_poses(la, mode, d_geno, n, d_ene, d_grad);
+    if (e == hipSuccess) e = launch_eval_poses(la, mode, d_geno, kGenes, n, d_ene, d_grad);
     if (e == hipSuccess && energies && mode != ADGPU_EVAL_GRADIENT)
         e = hipMemcpyAsync(energies, d_ene, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost, la.stream);
     if (e == hipSuccess && grads && mode != ADGPU_EVAL_ENERGY)
@@ -88,11 +89,11 @@ size_t lds_bytes(const LigandDev& Lh, int team_hint, int* team_width) {
     return s.lds;
 }
 
-hipError_t launch_eval_poses(const LaunchArgs& la, int mode, const float* genotypes, int n, float* energies,
-                             float* grads) {
+hipError_t launch_eval_poses(const LaunchArgs& la, int mode, const float* genotypes, int stride, int n,
+                             float* energies, float* grads) {
     if (n <= 0) return hipSuccess;
     Launch a{};
-    a.L = la.lig_dev; a.G = la.grid; a.in_geno = genotypes; a.out_e = energies; a.out_g = grads; a.n = n;
+    a.L = la.lig_dev; a.G = la.grid; a.in_geno = genotypes; a.stride = stride; a.out_e = energies; a.out_g = grads; a.n = n;
     a.mode = mode;
     const Shape sh = choose_shape(*la.lig_host, la.team_hint, true);
     const int per_group = 256 / sh.tw;

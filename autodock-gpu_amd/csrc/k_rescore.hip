@@ -38,7 +38,7 @@ DEV double wave_sum_d(double v) {
 }  // namespace
 
 template <int MF>
-__global__ __launch_bounds__(64) void k_rescore_f64(const LigandDev* L, GridDev G, const float* geno, int n,
+__global__ __launch_bounds__(64) void k_rescore_f64(const LigandDev* L, GridDev G, const float* geno, int stride, int n,
                                                     double* out3) {
     __shared__ double cx[ADGPU_MAX_ATOMS], cy[ADGPU_MAX_ATOMS], cz[ADGPU_MAX_ATOMS];
     const int pose = blockIdx.x;
@@ -54,7 +54,7 @@ __global__ __launch_bounds__(64) void k_rescore_f64(const LigandDev* L, GridDev 
     const PairB* pb = reinterpret_cast<const PairB*>(gb + L->off_pair_b);
     const PairX* px = reinterpret_cast<const PairX*>(gb + L->off_pair_x);
     const float2* tds = reinterpret_cast<const float2*>(gb + L->off_type_ds);
-    const float* g = geno + (size_t)pose * kGenes;
+    const float* g = geno + (size_t)pose * stride;
     const double d2r = (double)kDegToRad;
     const int N = L->num_atoms, P = L->num_pairs;
 
@@ -157,20 +157,20 @@ __global__ __launch_bounds__(64) void k_rescore_f64(const LigandDev* L, GridDev 
     }
 }
 
-hipError_t launch_rescore_f64(const LaunchArgs& la, const float* genotypes, int n, double* out3) {
+hipError_t launch_rescore_f64(const LaunchArgs& la, const float* genotypes, int stride, int n, double* out3) {
     if (n <= 0) return hipSuccess;
     switch (la.grid.format) {
         case ADGPU_MAP_F16:
             hipLaunchKernelGGL(k_rescore_f64<ADGPU_MAP_F16>, dim3(n), dim3(64), 0, la.stream, la.lig_dev, la.grid,
-                               genotypes, n, out3);
+                               genotypes, stride, n, out3);
             break;
         case ADGPU_MAP_BF16:
             hipLaunchKernelGGL(k_rescore_f64<ADGPU_MAP_BF16>, dim3(n), dim3(64), 0, la.stream, la.lig_dev, la.grid,
-                               genotypes, n, out3);
+                               genotypes, stride, n, out3);
             break;
         default:
             hipLaunchKernelGGL(k_rescore_f64<ADGPU_MAP_F32>, dim3(n), dim3(64), 0, la.stream, la.lig_dev, la.grid,
-                               genotypes, n, out3);
+                               genotypes, stride, n, out3);
     }
     return hipGetLastError();
 }
