@@ -47,6 +47,7 @@ struct LigandSet {
 // poses, else in parts of kStagePoses, kStageParts of them in flight.
 constexpr int kStageWhole = 8192, kStagePoses = 4096, kStageThreads = 4, kStageParts = 2 * kStageThreads;
 constexpr size_t kStageOpen = 512 * 1024;   // bytes of it that a context opens with
+constexpr int kMaxLanes = 4;
 
 struct adgpu_context {
     int device = 0;
@@ -67,6 +68,12 @@ struct adgpu_context {
     char* stage = nullptr;
     size_t stage_bytes = 0;
     hipEvent_t stage_ev[kStageParts] = {};
+    // streams that were seen to run side by side, for the run groups of one job
+    // at a time (make_lanes); more jobs at once make streams of their own
+    hipStream_t lane[kMaxLanes] = {};
+    int lanes = 0;
+    bool lanes_made = false;
+    std::atomic<bool> lanes_taken{false};
     float* noalloc = nullptr;  // this device's staging area of adgpu_eval_poses_noalloc
 };
 
@@ -78,6 +85,7 @@ constexpr int kRing = 16;   // generations a group may have in flight
 struct RunGroup {
     int r0 = 0, r1 = 0;                 // runs [r0, r1)
     hipStream_t stream = nullptr;
+    bool lent = false;                  // the stream is one of the context's lanes
     int parity = 0;                     // current population in buffer A (0) or B (1)
     int parity0 = 0;                    // parity when the current adgpu_job_run started
     int64_t done = 0, enq = 0;          // generations completed / enqueued in this adgpu_job_run
@@ -104,6 +112,7 @@ struct adgpu_job {
     adgpu_context* ctx = nullptr;
     int map_id = 0, ligand_id = 0;
     bool counted = false;               // holds a use of its maps and ligand
+    bool has_lanes = false;             // its groups run on the context's lanes
     // capacities of the device buffers; a serving slot reuses them for the
     // next request and grows them only when a request needs more
     size_t cap_ne = 0, cap_ls = 0;
@@ -600,6 +609,7 @@ int adgpu_close(adgpu_ctx c) {
     (void)hipStreamSynchronize(c->stream);
     for (auto& kv : c->maps) (void)hipFree(kv.second.data);
     for (auto& kv : c->ligands) (void)hipFree(kv.second.dev);
+    for (int k = 0; k < c->lanes; ++k) (void)hipStreamDestroy(c->lane[k]);
     if (c->stage) (void)hipHostFree(c->stage);
     for (hipEvent_t e : c->stage_ev)
         if (e) (void)hipEventDestroy(e);
@@ -833,9 +843,39 @@ int adgpu_rescore_f64(adgpu_ctx c, int map_id, int lig_id, const float* genotype
     return ADGPU_OK;
 }
 
+// Makes the context's lanes: up to kMaxLanes streams on hardware queues of
+// their own.  The runtime spreads a process's streams over its hardware
+// queues (GPU_MAX_HW_QUEUES, four unless set) by a rule of its own, and
+// kernels of streams that share a queue run one after the other: the docking
+// of 30 atoms, ADADELTA nrun 100, took 345 ms in four groups with three
+// contexts open and 600 ms with one, in two groups 385 and 600 ms with one and
+// two.  So streams are made one by one and kept when they are seen to run
+// beside the kept ones; those that do not stay until the end, so that the next
+// falls elsewhere.  Some 0.1 ms a stream, once per context; the context is held.
+static int make_lanes(adgpu_context* c) {
+    c->lanes_made = true;
+    hipStream_t spare[3 * kMaxLanes] = {};
+    int spares = 0;
+    hipError_t e = hipSuccess;
+    while (c->lanes < kMaxLanes && spares < 3 * kMaxLanes && e == hipSuccess) {
+        hipStream_t s = nullptr;
+        bool apart = false;
+        e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+        if (e != hipSuccess) break;
+        e = streams_overlap(s, c->lane, c->lanes, reinterpret_cast<uint64_t*>(c->stage), &apart);
+        if (e == hipSuccess && apart) c->lane[c->lanes++] = s;
+        else spare[spares++] = s;
+    }
+    for (int k = 0; k < spares; ++k) (void)hipStreamDestroy(spare[k]);
+    HIPCHK(c, e);
+    return ADGPU_OK;
+}
+
 // Run groups: streams and their per-generation events.
-static bool make_group(RunGroup& g) {
-    bool ok = hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking) == hipSuccess;
+static bool make_group(RunGroup& g, hipStream_t lane) {
+    bool ok = true;
+    if (lane) { g.stream = lane; g.lent = true; }
+    else ok = hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking) == hipSuccess;
     for (int r = 0; r < kRing && ok; ++r)
         ok = hipEventCreateWithFlags(&g.ev_done[r], g_wait_event_flags.load()) == hipSuccess &&
              hipEventCreate(&g.ev_gen[0][r]) == hipSuccess && hipEventCreate(&g.ev_gen[1][r]) == hipSuccess &&
@@ -853,7 +893,7 @@ static void drop_blocks(RunGroup& g) {
 static void destroy_group(RunGroup& g) {
     if (g.stream) (void)hipStreamSynchronize(g.stream);
     drop_blocks(g);   // before the stream its blocks were launched on
-    if (g.stream) (void)hipStreamDestroy(g.stream);
+    if (g.stream && !g.lent) (void)hipStreamDestroy(g.stream);
     for (int r = 0; r < kRing; ++r) {
         if (g.ev_done[r]) (void)hipEventDestroy(g.ev_done[r]);
         for (int h = 0; h < 2; ++h) {
@@ -875,7 +915,9 @@ static int job_set_groups(adgpu_job* j, int ng, int nrun) {
     }
     while ((int)j->groups.size() < ng) {
         j->groups.emplace_back();
-        if (!make_group(j->groups.back())) return fail(j->ctx, ADGPU_ERR_NOMEM, "stream or event creation failed");
+        const size_t k = j->groups.size() - 1;
+        if (!make_group(j->groups.back(), j->has_lanes && (int)k < j->ctx->lanes ? j->ctx->lane[k] : nullptr))
+            return fail(j->ctx, ADGPU_ERR_NOMEM, "stream or event creation failed");
     }
     for (int k = 0; k < ng; ++k) {
         j->groups[k].r0 = (int)((int64_t)nrun * k / ng);
@@ -1052,9 +1094,9 @@ int adgpu_job_create(adgpu_ctx c, int map_id, int lig_id, const adgpu_search_par
     j->ligand_id = lig_id;
     const int nrun = sp->num_runs;
     // run groups: ADGPU_RUN_GROUPS streams.  Groups whose streams share a
-    // hardware queue serialize, so there are at most four, with the HIP
-    // runtime's four hardware queues per process (GPU_MAX_HW_QUEUES) or more,
-    // and two with fewer.  A group's local-search launch should still fill a
+    // hardware queue serialize, so there are as many as the context has lanes
+    // (four with the HIP runtime's four hardware queues or more), and two when
+    // another job has them.  A group's local-search launch should still fill a
     // good part of the device, so small jobs get fewer groups: one per
     // kGroupSearches searches of a generation.  Launches in workgroups above
     // 256 threads (large pair lists) overlap worse: two groups.  ms a docking
@@ -1062,12 +1104,16 @@ int adgpu_job_create(adgpu_ctx c, int map_id, int lig_id, const adgpu_search_par
     // 52 / 59; Solis-Wets nrun 50, 30 atoms 72 / 59 / 60 / 58; ADADELTA nrun
     // 100, 23 atoms 64 / 57 / 57 / 52, 30 atoms - / 364 / 369 / 346; ADAM nrun
     // 50, 41 atoms - / 116 / 116 / 111; ADADELTA nrun 50, 54 atoms (512
-    // threads) - / 186 / 195 / 191.  Six groups on four queues: twice the time
-    // of two.
-    int ng = 4;
-    if (const char* q = std::getenv("GPU_MAX_HW_QUEUES"))
-        if (std::atoi(q) >= 1 && std::atoi(q) < 4) ng = 2;
+    // threads) - / 186 / 195 / 191.
+    int ng = 2;
     const int64_t searches = (int64_t)nrun * std::max(1, to_dev(sp, num_genes).num_ls);
+    const bool several = searches >= 2 * kGroupSearches || std::getenv("ADGPU_RUN_GROUPS");
+    if (several && !c->lanes_made)
+        if (int rc = make_lanes(c)) return rc;
+    if (several && c->lanes > 1 && !c->lanes_taken.exchange(true)) {
+        j->has_lanes = true;   // until the job is destroyed
+        ng = c->lanes;
+    }
     ng = (int)std::max<int64_t>(1, std::min<int64_t>(ng, searches / kGroupSearches));
     if (ng > 2) {
         const int tw = job_team_width(c, li->second.host.num_atoms, searches, 1, sp->ls_method);
@@ -1104,6 +1150,7 @@ int adgpu_job_destroy(adgpu_job_t j) {
         if (!j->own_lig && li != j->ctx->ligands.end()) li->second.jobs--;
     }
     for (auto& g : j->groups) destroy_group(g);
+    if (j->has_lanes) j->ctx->lanes_taken = false;
     (void)hipFree(j->pop[0]); (void)hipFree(j->pop[1]);
     (void)hipFree(j->ene[0]); (void)hipFree(j->ene[1]);
     (void)hipFree(j->evals_new); (void)hipFree(j->evals_runs); (void)hipFree(j->prng);

@@ -32,7 +32,37 @@ __global__ __launch_bounds__(256) void k_valu_rate(float* out, int iters, float 
     out[blockIdx.x * blockDim.x + threadIdx.x] = s;
 }
 
+// Stays on the device for `ticks` of the 100 MHz clock (bounded by the trip
+// count) and leaves the times it began and ended.
+__global__ __launch_bounds__(64) void k_hold(uint64_t* span, uint32_t ticks) {
+    const uint64_t begin = wall_clock64();
+    uint64_t now = begin;
+    for (int i = 0; i < 20000 && now - begin < ticks; ++i) {
+        __builtin_amdgcn_s_sleep(1);
+        now = wall_clock64();
+    }
+    if (threadIdx.x == 0) { span[0] = begin; span[1] = now; }
+}
+
 }  // namespace
+
+hipError_t streams_overlap(hipStream_t s, const hipStream_t* others, int n, uint64_t* span, bool* all) {
+    *all = false;
+    // the first launch on a stream may wait for its queue: once before the test
+    for (int round = 0; round < 2; ++round) {
+        hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, s, span, round ? 6000u : 10u);
+        for (int k = 0; k < n; ++k)
+            hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, others[k], span + 2 + 2 * k, 10u);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        for (int k = 0; k < n && e == hipSuccess; ++k) e = hipStreamSynchronize(others[k]);
+        if (e != hipSuccess) return e;
+    }
+    bool ok = true;
+    for (int k = 0; k < n; ++k) ok = ok && span[2 + 2 * k] < span[1];
+    *all = ok;
+    return hipSuccess;
+}
 
 hipError_t measure_valu_rate(hipStream_t stream, float* scratch, int blocks, int iters, double* wave_instr_per_s) {
     hipEvent_t e0 = nullptr, e1 = nullptr;

@@ -231,3 +231,38 @@ def test_maps_and_ligand_outlive_their_jobs(gpu_ctx):
     job.destroy()
     gpu_ctx.ligand_release(lid)
     gpu_ctx.maps_release(mid)
+
+
+def test_jobs_share_a_contexts_lanes(gpu_ctx, c1):
+    """Jobs of several run groups alive at once on one context: the first takes
+    the context's streams, the others make their own; whichever goes first,
+    each docks as it does alone."""
+    mid = gpu_ctx.maps_upload(c1.packed, c1.size, c1.maps.num_map_atypes, c1.spacing)
+    lid = gpu_ctx.ligand_upload(c1.tables, c1.ep)
+    sp = search_params(num_runs=40, pop_size=100, max_evals=20000, ls="ad", spacing=c1.spacing, max_iters=30)
+
+    def job(k):
+        init = O.initial_population((k,), 40, 100, c1.maps.size_angstr, c1.spacing)
+        return gpu_ctx.job(mid, lid, sp, init, O.cmwc_uints((k,), 40 * 100 * 64))
+
+    def docked(j):
+        j.initpop()
+        return j.run(), j.download()
+
+    alone = []
+    for k in (1, 2, 3):
+        j = job(k)
+        alone.append(docked(j))
+        j.destroy()
+    a, b = job(1), job(2)
+    got = [docked(a), docked(b)]
+    a.destroy()
+    c = job(3)          # on the streams that the first gave back
+    got.append(docked(c))
+    b.destroy()
+    c.destroy()
+    for (r0, d0), (r1, d1) in zip(alone, got):
+        assert r0 == r1
+        assert np.array_equal(d0["pop"], d1["pop"]) and np.array_equal(d0["ene"], d1["ene"])
+    gpu_ctx.ligand_release(lid)
+    gpu_ctx.maps_release(mid)
