@@ -126,3 +126,31 @@ def test_run_stops_where_the_host_loop_stops(gpu_ctx, c1g, ls, stopstd, min_frac
         assert np.array_equal(a.download()["pop"], sa["pop"])
     a.destroy()
     b.destroy()
+
+
+@pytest.mark.parametrize("nrun,pop", [(1, 2), (13, 157), (16, 128), (17, 121), (2, 700), (5, 2048)])
+def test_records_at_the_edges_of_chunks_and_bins(gpu_ctx, c1g, nrun, pop):
+    """Sample counts around one chunk of energies (2041, 2048, 2057) and over
+    several, more bins than one pass of the bins' lanes takes, the smallest
+    population; energies equal, of both zeros, infinite and NaN among them."""
+    rng = np.random.default_rng(nrun * pop)
+    job = _job(gpu_ctx, c1g, nrun, pop, ls="sw")
+    job.initpop()
+    asf = 2
+    job.set_autostop(True, stopstd=0.15, as_frequency=asf, min_as_evals=10 ** 12)
+    orc = O.OracleAutoStop(pop, nrun, 0.15, asf)
+    for c in range(4):
+        e = np.round(rng.normal(-3 - c, 2.0 / (1 + c), nrun * pop), 2).astype(np.float32)
+        e[:: 5] = e.min()                                  # the lowest bin takes a fifth of the samples
+        if e.size > 100:
+            e[7], e[11], e[13], e[17] = np.inf, np.nan, 0.0, -0.0
+        if c:
+            for _ in range(asf):
+                job.sum_and_swap()
+        job.upload(ene=e)
+        rec = job.autostop_check()
+        total = nrun * pop * (1 + asf * c)
+        _, ref = orc.check(c * asf, e, total, 10 ** 12)
+        _same_record(rec, ref, c)
+    _same_record(job.autostop_final(), orc.final(asf * 3, e, total), "final")
+    job.destroy()
