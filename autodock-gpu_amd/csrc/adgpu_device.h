@@ -1136,9 +1136,9 @@ struct Launch {
     EvalCtx<TW, NC> X;                                                         \
     X.L = a.L;                                                                 \
     X.G = a.G;                                                                 \
-    stage<TW, NC, PL, GRAD>(a.L, lds, X.sv, X.tv);                                 \
-    X.A.load(a.L, a.G);                                                        \
+    X.A.load(a.L, a.G);   /* its loads run beside the staging's */              \
     X.ls.load(a.L);                                                            \
+    stage<TW, NC, PL, GRAD>(a.L, lds, X.sv, X.tv);                             \
     const int tl = TM::lane();                                                 \
     (void)tl;                                                                  \
     const int team_idx = (int)(blockIdx.x * (blockDim.x / TW) + threadIdx.x / TW); \

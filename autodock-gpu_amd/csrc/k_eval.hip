@@ -12,13 +12,18 @@ namespace adgpu {
 // nothing, so every wavefront runs the evaluation with all lanes.
 template <int TW, int NC, int MF, bool PL>
 __global__ ADGPU_GROUP_KERNEL void k_eval_poses(Launch a) {
+    // the genotype first: in pinned host memory it takes longest to arrive
+    float gene[64 / TW], grad[64 / TW];
+    const int pose = min((int)(blockIdx.x * (blockDim.x / TW) + threadIdx.x / TW), a.n - 1);
+#pragma unroll
+    for (int j = 0; j < 64 / TW; ++j) {
+        const int g = Team<TW>::lane() + TW * j;
+        gene[j] = g < a.stride ? a.in_geno[(size_t)pose * a.stride + g] : 0.f;
+    }
     KERNEL_PROLOGUE(TW, NC, PL, true)
     const bool live = team_idx < a.n;
     if (!TM::any_in_wave(live)) return;
-    const int id = live ? team_idx : a.n - 1;
-    float gene[GPL], grad[GPL];
-#pragma unroll
-    for (int j = 0; j < GPL; ++j) gene[j] = tl + TW * j < a.stride ? a.in_geno[(size_t)id * a.stride + tl + TW * j] : 0.f;
+    const int id = pose;
     if (a.mode == ADGPU_EVAL_GRADIENT) {
         float_gradient<TW, NC, MF, PL>(X, gene, grad);
     } else if (a.mode == ADGPU_EVAL_ENERGRAD) {
