@@ -196,6 +196,19 @@ DEV float3 qrot(float3 v, float4 q) {
                        v.z + zz * q.w + (q.x * zy - q.y * zx));
 }
 
+// The same bits with q2 = (2 q.x, 2 q.y, 2 q.z, q.w): both cross products come
+// out doubled, which is exact, the first as it is needed and the second halved
+// by the addition that takes it -- three additions less.
+DEV float3 qrot2(float3 v, float4 q2) {
+#pragma clang fp contract(off)
+    const float zx = fmaf(q2.y, v.z, -(q2.z * v.y));
+    const float zy = fmaf(q2.z, v.x, -(q2.x * v.z));
+    const float zz = fmaf(q2.x, v.y, -(q2.y * v.x));
+    return make_float3(fmaf(0.5f, fmaf(q2.y, zz, -(q2.z * zy)), fmaf(zx, q2.w, v.x)),
+                       fmaf(0.5f, fmaf(q2.z, zx, -(q2.x * zz)), fmaf(zy, q2.w, v.y)),
+                       fmaf(0.5f, fmaf(q2.x, zy, -(q2.y * zx)), fmaf(zz, q2.w, v.z)));
+}
+
 // quaternion_multiply, calcenergy.cl:110-117
 DEV float4 qmul(float4 a, float4 b) {
     return make_float4(a.w * b.x + a.x * b.w + a.y * b.z - a.z * b.y,
@@ -459,16 +472,17 @@ struct EvalCtx {
 // ligand block instead of keeping a register.
 template <int TW, int NC, class F>
 DEV void for_bonds(const EvalCtx<TW, NC>& X, int k, float4 TorRec::*second, F&& f) {
-    const TorRec* tor = X.tv.tor;
     const int T = X.ls.T;
+    // a 24-bit product: 64-bit address arithmetic takes four times as long
+    auto rec = [&](int t) { return at(X.tv.tor, __umul24((uint32_t)t, (uint32_t)sizeof(TorRec))); };
     if (uint32_t m = X.A.mlo[k]) {
         int t = __builtin_ctz(m);
-        float4 q = tor[t].q, v = tor[t].*second;
+        float4 q = rec(t)->q, v = rec(t)->*second;
         for (;;) {
             m &= m - 1;
             if constexpr (TW == 64) {
                 const int next = m ? __builtin_ctz(m) : t;
-                const float4 nq = tor[next].q, nv = tor[next].*second;
+                const float4 nq = rec(next)->q, nv = rec(next)->*second;
                 f(t, q, v);
                 if (!m) break;
                 t = next; q = nq; v = nv;
@@ -476,7 +490,7 @@ DEV void for_bonds(const EvalCtx<TW, NC>& X, int k, float4 TorRec::*second, F&& 
                 f(t, q, v);
                 if (!m) break;
                 t = __builtin_ctz(m);
-                q = tor[t].q; v = tor[t].*second;
+                q = rec(t)->q; v = rec(t)->*second;
             }
         }
     }
@@ -486,7 +500,7 @@ DEV void for_bonds(const EvalCtx<TW, NC>& X, int k, float4 TorRec::*second, F&& 
         uint32_t m = X.A.valid[k] ? am[Team<TW>::lane() + TW * k].y : 0u;
         for (; m; m &= m - 1) {
             const int t = 32 + __builtin_ctz(m);
-            f(t, tor[t].q, tor[t].*second);
+            f(t, rec(t)->q, rec(t)->*second);
         }
     }
 }
@@ -524,7 +538,8 @@ DEV void gene_trig(const LigScalars& ls, const SharedView& sv, const TeamView& t
                 tv.pg[7 + 2 * (g - 3)] = c;
             } else {
                 float4 u = sv.tor_unit[g - 6];
-                tv.tor[g - 6].q = make_float4(s * u.x, s * u.y, s * u.z, c);
+                s += s;
+                tv.tor[g - 6].q = make_float4(s * u.x, s * u.y, s * u.z, c);   // as qrot2 takes it
             }
         }
     }
@@ -563,7 +578,7 @@ DEV void compute_coords(const EvalCtx<TW, NC>& X, const Pose& P, float3 (&c)[NC]
     for (int k = 0; k < NC; ++k) {
         float3 v = A.ref[k];
         for_bonds<TW, NC>(X, k, &TorRec::m, [&](int, const float4& q, const float4& m) {
-            float3 r = qrot(make_float3(v.x - m.x, v.y - m.y, v.z - m.z), q);
+            float3 r = qrot2(make_float3(v.x - m.x, v.y - m.y, v.z - m.z), q);
             v = make_float3(r.x + m.x, r.y + m.y, r.z + m.z);
         });
         if (A.lig[k]) {
@@ -637,13 +652,13 @@ DEV float gather_finish(const GridDev& G, float3 c, float q, const Gather<MF>& g
     const float y0 = omdy * x00 + dy * x10, y1 = omdy * x01 + dy * x11;
     const float e = omdz * y0 + dz * y1;
     if (GRAD) {
-        const float ig = G.inv_spacing;
+        const float ig = kTermScale * G.inv_spacing;   // a power of two: the same rounded products
         const float gx = omdz * (omdy * (h.x - l.x) + dy * (h.y - l.y)) + dz * (omdy * (h.z - l.z) + dy * (h.w - l.w));
         const float gy = omdz * (x10 - x00) + dz * (x11 - x01);
         const float gz = y1 - y0;
-        fi.x += quant(kTermScale * (gx * ig));
-        fi.y += quant(kTermScale * (gy * ig));
-        fi.z += quant(kTermScale * (gz * ig));
+        fi.x += quant(gx * ig);
+        fi.y += quant(gy * ig);
+        fi.z += quant(gz * ig);
     }
     return e;
 }
@@ -658,9 +673,10 @@ DEV float gather_finish(const GridDev& G, float3 c, float q, const Gather<MF>& g
 // dist = distance in grid units, rdist = 1 / dist, inv_sp = 1 / spacing: 1/r in
 // A is rdist * inv_sp unless r is clamped at elec_min_distance.  Every fused
 // multiply-add is written out, so all kernels round alike.
-template <bool GRAD>
-DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, const PairX* px, float spacing,
-                      float dist, float rdist, float inv_sp, float& dedr) {
+// flags(): the pair's PairX::flags.
+template <bool GRAD, class F>
+DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, F&& flags, float spacing, float dist,
+                      float rdist, float inv_sp, float& dedr) {
 #pragma clang fp contract(off)
     // vdW / H-bond with smoothing, r < 8 A: with qm = sd^-m and qn = sd^-n,
     // E = AC qm - BD qn and dE/dsd = -(m AC qm - n BD qn) / sd.  sd^-12 is one
@@ -677,7 +693,7 @@ DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, co
     float evdw = fmaf(pa.ac, qm, -bn);
     float dvdw = GRAD ? fmaf(bn, pa.fn, -(12.0f * am)) * q : 0.0f;
     if (__builtin_expect(ls.any_general, 0)) {        // other exponents (modified pairs): rare,
-        const uint32_t fl = px->flags;                // kept off the common path
+        const uint32_t fl = flags();                  // kept off the common path
         if (!(fl & kPairFast)) {
             const float fm = (float)(fl & 0xffu);
             const float l2 = __builtin_amdgcn_logf(sd);
@@ -763,7 +779,6 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
     float e = 0.f;
     const PairA* ra = sv.pa + tl;
     const PairB* rb = sv.pb + tl;
-    const PairX* rx = sv.px + tl;
     // Every lane has a record in every step (padding), so the loop count is
     // uniform: no execution masks, and the counter is scalar.  With the atoms
     // kept as byte offsets, the exponent as a float, the two halves of a step
@@ -801,7 +816,11 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
         const float rdist = fast_rsq(d2g);            // one transcendental for r and 1/r
         const float dist = d2g * rdist;
         float dedr;
-        e += pair_energy<GRAD>(X.ls, pa, pb, rx, spacing, dist, rdist, G.inv_spacing, dedr);
+        auto flags = [&] {
+            const uint32_t at = (uint32_t)(ra - sv.pa);
+            return sv.px[PL ? (at + tl) >> 1 : at].flags;   // in LDS a step's records are TW PairA apart
+        };
+        e += pair_energy<GRAD>(X.ls, pa, pb, flags, spacing, dist, rdist, G.inv_spacing, dedr);
         if (GRAD) {
             // TERMSCALE * s * gdd with the power-of-two scale folded into gdd:
             // the same rounded product
@@ -813,7 +832,6 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
         if constexpr (!PL) { pa = pa_next; pb = pb_next; }
         ra += pair_stride<TW, PL>;
         rb += pair_stride<TW, PL>;
-        rx += TW;
     }
     int3 fi[NC];
 #pragma unroll
@@ -908,7 +926,7 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
             const float qx = ry * F[k].z - rz * F[k].y, qy = rz * F[k].x - rx * F[k].z,
                         qz = rx * F[k].y - ry * F[k].x;
             const float toa = (ax.x * qx + ax.y * qy + ax.z * qz) * spacing;
-            atomicAdd(&tv.gi[4 * t + (tl & 3)], quant(kTermScale * toa * kDegToRad));
+            atomicAdd(&tv.gi[4 * t + (tl & 3)], quant(toa * (kTermScale * kDegToRad)));
         });
     }
     wave_sync();
@@ -923,8 +941,7 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
             const int4 part = reinterpret_cast<const int4*>(tv.gi)[g - 6];
             iv = part.x + part.y + part.z + part.w;
         }
-        float gv = kOneOverTermScale * (float)iv;
-        if (g >= 3) gv *= conv;
+        const float gv = (float)iv * (g >= 3 ? kOneOverTermScale * conv : kOneOverTermScale);
         grad[j] = g < NG ? gv : 0.f;
     }
     return energy;
