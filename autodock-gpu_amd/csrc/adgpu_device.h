@@ -276,9 +276,22 @@ struct TorRec {
     float4 r0;
 };
 
+// A pair's record as the energy takes it.
+struct PairRec {
+    uint32_t ij;
+    float fn, ac, bd, reqm, cq, dsol, g;
+};
+DEV PairRec unpack(const PairA& a, const PairB& b) {
+    return PairRec{a.ij, a.fn, a.ac, a.bd, b.reqm, b.cq, b.dsol, b.g};
+}
+DEV PairRec unpack(const PairC& c) {   // g: with the flags
+    return PairRec{c.ij & ~kPairTen, (int)c.ij < 0 ? 10.0f : 6.0f, c.ac, c.bd, c.reqm, c.cq, c.dsol, 0.0f};
+}
+
 struct SharedView {           // staged once per workgroup
     const PairA* pa;          // LDS (or global when the pairs do not fit): record p of step k is
     const PairB* pb;          //   [k * pair_stride<TW, PL> + lane] of both
+    const PairC* pc;          // in place of pa and pb (compact_pairs)
     const PairX* px;          // global (rarely read)
     const float4* tor_unit;
     const int2* tor_atoms;
@@ -310,8 +323,8 @@ __host__ __device__ inline size_t align16(size_t x) { return (x + 15) & ~size_t(
 template <int TW, bool PL>
 constexpr int pair_stride = PL ? 2 * TW : TW;
 
-__host__ __device__ inline size_t shared_bytes_for(int TW, int T, int P, bool pairs_in_lds) {
-    size_t s = pairs_in_lds ? (size_t)padded_pairs(P, TW) * (sizeof(PairA) + sizeof(PairB)) : 0;
+__host__ __device__ inline size_t shared_bytes_for(int TW, int NC, int T, int P, bool pairs_in_lds, bool GRAD) {
+    size_t s = pairs_in_lds ? (size_t)padded_pairs(P, TW) * (compact_pairs(TW * NC, GRAD) ? sizeof(PairC) : sizeof(PairA) + sizeof(PairB)) : 0;
     s += (size_t)T * (sizeof(float4) + sizeof(int2));
     return align16(s);
 }
@@ -333,7 +346,7 @@ __host__ __device__ inline size_t team_bytes_for(int TW, int NC, int T, bool PL,
 
 // LDS of one workgroup of `threads` threads (threads / TW teams).
 __host__ __device__ inline size_t lds_bytes_for(int TW, int NC, int T, int P, bool PL, bool GRAD, int threads) {
-    return shared_bytes_for(TW, T, P, PL) + (size_t)(threads / TW) * team_bytes_for(TW, NC, T, PL, GRAD);
+    return shared_bytes_for(TW, NC, T, P, PL, GRAD) + (size_t)(threads / TW) * team_bytes_for(TW, NC, T, PL, GRAD);
 }
 
 // Stages the shared tables (all threads of the workgroup) and carves the
@@ -347,7 +360,16 @@ DEV void stage(const LigandDev* L, char* lds, SharedView& sv, TeamView& tv) {
     const PairA* gpa = reinterpret_cast<const PairA*>(gbase + L->off_pair_a[slot_copies(TW, NC) - 1]);
     const PairB* gpb = reinterpret_cast<const PairB*>(gbase + L->off_pair_b);
     sv.px = reinterpret_cast<const PairX*>(gbase + L->off_pair_x);
-    if (PL) {
+    constexpr bool kCompact = compact_pairs(TW * NC, GRAD);
+    sv.pc = reinterpret_cast<const PairC*>(gbase + L->off_pair_c);
+    if constexpr (PL && kCompact) {
+        static_assert(slot_copies(TW, NC) == 1, "staged as it is stored");
+        const int PP = padded_pairs(P, TW);
+        PairC* lc = reinterpret_cast<PairC*>(p);
+        for (int k = threadIdx.x; k < PP; k += blockDim.x) lc[k] = sv.pc[k];
+        sv.pc = lc;
+        p += (size_t)PP * sizeof(PairC);
+    } else if (PL) {
         const int PP = padded_pairs(P, TW);
         PairA* la = reinterpret_cast<PairA*>(p);
         PairB* lb = reinterpret_cast<PairB*>(la + TW);
@@ -376,7 +398,7 @@ DEV void stage(const LigandDev* L, char* lds, SharedView& sv, TeamView& tv) {
     const int2* gta = reinterpret_cast<const int2*>(gbase + L->off_tor_atoms);
     for (int k = threadIdx.x; k < T; k += blockDim.x) { tu[k] = gtu[k]; ta[k] = gta[k]; }
     sv.tor_unit = tu; sv.tor_atoms = ta;
-    char* w = lds + shared_bytes_for(TW, T, P, PL) + (size_t)(threadIdx.x / TW) * team_bytes_for(TW, NC, T, PL, GRAD);
+    char* w = lds + shared_bytes_for(TW, NC, T, P, PL, GRAD) + (size_t)(threadIdx.x / TW) * team_bytes_for(TW, NC, T, PL, GRAD);
     constexpr int kCoords = coord_array(TW, NC, PL, GRAD), kForces = slot_array(TW, NC);
     tv.cx = reinterpret_cast<float*>(w);
     tv.cy = tv.cx + kCoords;
@@ -674,8 +696,8 @@ DEV float gather_finish(const GridDev& G, float3 c, float q, const Gather<MF>& g
 // A is rdist * inv_sp unless r is clamped at elec_min_distance.  Every fused
 // multiply-add is written out, so all kernels round alike.
 // flags(): the pair's PairX::flags.
-template <bool GRAD, class F>
-DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, F&& flags, float spacing, float dist,
+template <bool GRAD, bool COMPACT, class F>
+DEV float pair_energy(const LigScalars& ls, const PairRec& pr, F&& flags, float spacing, float dist,
                       float rdist, float inv_sp, float& dedr) {
 #pragma clang fp contract(off)
     // vdW / H-bond with smoothing, r < 8 A: with qm = sd^-m and qn = sd^-n,
@@ -683,24 +705,26 @@ DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, F&
     // reciprocal of sd^12 (a few ulp; the 12th power of 1/sd would carry up to
     // 12 ulp), and sd^-n = sd^-12 sd^(12-n)
     const float ad = dist * spacing;
-    const float delta = fmaf(-spacing, dist, pb.reqm);
-    const float sd = (fabsf(delta) >= ls.half_smooth) ? fmaf(spacing, dist, copysignf(ls.half_smooth, delta)) : pb.reqm;
+    const float delta = fmaf(-spacing, dist, pr.reqm);
+    const float sd = (fabsf(delta) >= ls.half_smooth) ? fmaf(spacing, dist, copysignf(ls.half_smooth, delta)) : pr.reqm;
     const float r2 = sd * sd, r4 = r2 * r2, r6 = r4 * r2;
     const float qm = fast_rcp(r6 * r6);               // m = 12
-    const float qn = qm * (pa.fn == 6.0f ? r6 : r2);  // n = 6 or 10
+    const float qn = qm * (pr.fn == 6.0f ? r6 : r2);  // n = 6 or 10
     const float q = GRAD ? fast_rcp(sd) : 0.0f;
-    const float am = pa.ac * qm, bn = pa.bd * qn;
-    float evdw = fmaf(pa.ac, qm, -bn);
-    float dvdw = GRAD ? fmaf(bn, pa.fn, -(12.0f * am)) * q : 0.0f;
+    const float am = pr.ac * qm, bn = pr.bd * qn;
+    float evdw = fmaf(pr.ac, qm, -bn);
+    float dvdw = GRAD ? fmaf(bn, pr.fn, -(12.0f * am)) * q : 0.0f;
+    float g = pr.g;                                   // CG-G0 bond constant: 50 for a CG-G0 pair, else 0
     if (__builtin_expect(ls.any_general, 0)) {        // other exponents (modified pairs): rare,
         const uint32_t fl = flags();                  // kept off the common path
+        if (COMPACT && (fl & kPairCgG0)) g = 50.0f;
         if (!(fl & kPairFast)) {
-            const float fm = (float)(fl & 0xffu);
+            const float fm = (float)(fl & 0xffu), fn = (float)((fl >> 8) & 0xffu);
             const float l2 = __builtin_amdgcn_logf(sd);
             const float gm = __builtin_amdgcn_exp2f(-fm * l2);
-            const float ga = pa.ac * gm, gb = pa.bd * __builtin_amdgcn_exp2f(-pa.fn * l2);
-            evdw = fmaf(pa.ac, gm, -gb);
-            if (GRAD) dvdw = fmaf(gb, pa.fn, -(fm * ga)) * q;
+            const float ga = pr.ac * gm, gb = pr.bd * __builtin_amdgcn_exp2f(-fn * l2);
+            evdw = fmaf(pr.ac, gm, -gb);
+            if (GRAD) dvdw = fmaf(gb, fn, -(fm * ga)) * q;
         }
     }
     // electrostatics and desolvation, r < 20.48 A, r clamped at elec_min_distance:
@@ -709,19 +733,18 @@ DEV float pair_energy(const LigScalars& ls, const PairA& pa, const PairB& pb, F&
     const float d2 = d * d;
     const float num = fmaf(-0.1063f * d2, fmaf(-0.001947f, d2, 1.0f), 12.96f);
     const float den = fmaf(d2, fmaf(d2, fmaf(0.000112f, d2, 0.00357f), 0.4137f), 12.96f);
-    const float desolv = pb.dsol * (ls.coeff_desolv * num * fast_rcp(den));
+    const float desolv = pr.dsol * (ls.coeff_desolv * num * fast_rcp(den));
     const float rds = fast_rcp(d + 1.26366f);
     const float rds2 = rds * rds;
     const float diel = fmaf(1.10859f, rds2, 0.010358f);
     const float rd = min_s(rdist * inv_sp, ls.inv_elec_min);
-    const float es = pb.cq * rd;
+    const float es = pr.cq * rd;
     const float eel = fmaf(es, diel, desolv);
     const bool in8 = ad < 8.0f, in20 = ad < 20.48f;
-    // CG-G0 bond term, G = 50 (0 for other pairs)
-    const float e = fmaf(pb.g, ad, in8 ? evdw : 0.0f) + (in20 ? eel : 0.0f);
+    const float e = fmaf(g, ad, in8 ? evdw : 0.0f) + (in20 ? eel : 0.0f);
     if (GRAD) {
         const float del = fmaf(-0.0771605f * d, desolv, fmaf(rds, es * -2.21718f * rds2, -(es * rd * diel)));
-        dedr = pb.g + (in8 ? dvdw : 0.0f) + (in20 ? del : 0.0f);
+        dedr = g + (in8 ? dvdw : 0.0f) + (in20 ? del : 0.0f);
     } else {
         dedr = 0.f;
     }
@@ -777,8 +800,10 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
 
     const float spacing = G.spacing;
     float e = 0.f;
+    constexpr bool kCompact = compact_pairs(TW * NC, GRAD_KERNEL);
     const PairA* ra = sv.pa + tl;
     const PairB* rb = sv.pb + tl;
+    const PairC* rc = sv.pc + tl;
     // Every lane has a record in every step (padding), so the loop count is
     // uniform: no execution masks, and the counter is scalar.  With the atoms
     // kept as byte offsets, the exponent as a float, the two halves of a step
@@ -796,20 +821,23 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
     // evals/s with many, and is not done.
     PairA pa{};
     PairB pb{};
-    if (!PL && steps > 0) { pa = *ra; pb = *rb; }
+    PairC pc{};
+    if (!PL && steps > 0) {
+        if constexpr (kCompact) pc = *rc;
+        else { pa = *ra; pb = *rb; }
+    }
 #pragma unroll 1
     for (int k = 0; k < steps; ++k) {
         PairA pa_next{};
         PairB pb_next{};
-        if constexpr (PL) {
-            pa = *ra;
-            pb = *rb;
-        } else {
-            const int next = k + 1 < steps ? pair_stride<TW, PL> : 0;
-            pa_next = ra[next];
-            pb_next = rb[next];
-        }
-        const uint32_t io = pa.ij & 0xffffu, jo = pa.ij >> 16;
+        PairC pc_next{};
+        const int next = k + 1 < steps ? TW : 0;
+        if constexpr (PL && kCompact) pc = *rc;
+        else if constexpr (PL) { pa = *ra; pb = *rb; }
+        else if constexpr (kCompact) pc_next = rc[next];
+        else { pa_next = ra[next]; pb_next = rb[next]; }
+        const PairRec pr = kCompact ? unpack(pc) : unpack(pa, pb);
+        const uint32_t io = pr.ij & 0xffffu, jo = pr.ij >> 16;
         const float sx = *at(tv.cx, io) - *at(tv.cx, jo), sy = *at(tv.cy, io) - *at(tv.cy, jo),
                     sz = *at(tv.cz, io) - *at(tv.cz, jo);
         const float d2g = fmaf(sz, sz, fmaf(sx, sx, sy * sy));
@@ -817,10 +845,10 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
         const float dist = d2g * rdist;
         float dedr;
         auto flags = [&] {
-            const uint32_t at = (uint32_t)(ra - sv.pa);
-            return sv.px[PL ? (at + tl) >> 1 : at].flags;   // in LDS a step's records are TW PairA apart
+            const uint32_t at = kCompact ? (uint32_t)(rc - sv.pc) : (uint32_t)(ra - sv.pa);
+            return sv.px[PL && !kCompact ? (at + tl) >> 1 : at].flags;   // a step's records are TW PairA apart
         };
-        e += pair_energy<GRAD>(X.ls, pa, pb, flags, spacing, dist, rdist, G.inv_spacing, dedr);
+        e += pair_energy<GRAD, kCompact>(X.ls, pr, flags, spacing, dist, rdist, G.inv_spacing, dedr);
         if (GRAD) {
             // TERMSCALE * s * gdd with the power-of-two scale folded into gdd:
             // the same rounded product
@@ -829,9 +857,10 @@ DEV float evaluate(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], float
             lds_sub(at(tv.fx, io), ix); lds_sub(at(tv.fy, io), iy); lds_sub(at(tv.fz, io), iz);
             atomicAdd(at(tv.fx, jo), ix); atomicAdd(at(tv.fy, jo), iy); atomicAdd(at(tv.fz, jo), iz);
         }
-        if constexpr (!PL) { pa = pa_next; pb = pb_next; }
+        if constexpr (!PL) { pa = pa_next; pb = pb_next; pc = pc_next; }
         ra += pair_stride<TW, PL>;
         rb += pair_stride<TW, PL>;
+        rc += TW;
     }
     int3 fi[NC];
 #pragma unroll
@@ -1021,8 +1050,7 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
     const float DA = -8.5525f, DB = 78.4f - (-8.5525f), DK = 7.7839f;
     const float DBH = DB * 0.003627f, DBHK = DBH * DK;
     for (int p = tl, r = tl; p < P; p += TW, r += pair_stride<TW, PL>) {
-        const PairA pa = sv.pa[r];
-        const PairB pb = sv.pb[r];
+        const PairRec pr = compact_pairs(TW * NC, true) ? unpack(sv.pc[p]) : unpack(sv.pa[r], sv.pb[r]);
         // the pair's atoms in the list's order, first copies: float sums keep their order
         const uint32_t fl = sv.px[p].flags, atoms = sv.px[p].atoms;
         const int i = (int)(atoms & 0xffffu), j = (int)(atoms >> 16);
@@ -1030,14 +1058,14 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
         const float dist = sqrtf(sx * sx + sy * sy + sz * sz);
         float d = dist * spacing;
         float sd;
-        if (d <= pb.reqm - half_smooth) sd = d + half_smooth;
-        else if (d < pb.reqm + half_smooth) sd = pb.reqm;
+        if (d <= pr.reqm - half_smooth) sd = d + half_smooth;
+        else if (d < pr.reqm + half_smooth) sd = pr.reqm;
         else sd = d - half_smooth;
         const int m = (int)(fl & 0xffu), n = (int)((fl >> 8) & 0xffu);
         float pg = 0.f;
         if (d < 8.0f) {
-            pg += (-(float)m * pa.ac) / powf(sd, (float)(m + 1));
-            pg += ((float)n * pa.bd) / powf(sd, (float)(n + 1));
+            pg += (-(float)m * pr.ac) / powf(sd, (float)(m + 1));
+            pg += ((float)n * pr.bd) / powf(sd, (float)(n + 1));
         }
         if (d < 20.48f) {
             if (d < X.ls.elec_min) d = X.ls.elec_min;
@@ -1045,8 +1073,8 @@ DEV void float_gradient(const EvalCtx<TW, NC>& X, const float (&gene)[64 / TW], 
             const float upper = DA * (ex + DK) * (ex + DK) + DB * ex * (DBHK * d + ex + DK);
             const float lw = DA * (ex + DK) + DB * ex;
             const float lower = d * d * lw * lw;
-            pg += -pb.cq * (upper / lower);
-            pg += pb.dsol * X.ls.coeff_desolv * -0.077160f * d * __expf(-0.038580f * d * d);
+            pg += -pr.cq * (upper / lower);
+            pg += pr.dsol * X.ls.coeff_desolv * -0.077160f * d * __expf(-0.038580f * d * d);
         }
         if (fl & kPairCgG0) pg += 50.0f;
         const float fx = pg * (-sx / dist), fy = pg * (-sy / dist), fz = pg * (-sz / dist);

@@ -382,6 +382,7 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
     if (one) hd.off_pair_a[0] = take(sizeof(PairA) * (P ? PP : 1));
     if (two) hd.off_pair_a[1] = take(sizeof(PairA) * (P ? PP : 1));
     hd.off_pair_b = take(sizeof(PairB) * (P ? PP : 1));
+    if (N > kFullPairAtoms) hd.off_pair_c = take(sizeof(PairC) * (P ? PP : 1));
     hd.off_pair_x = take(sizeof(PairX) * (P ? PP : 1));
     hd.off_type_ds = take(sizeof(float2) * NT);
     hd.total_bytes = (uint32_t)off;
@@ -437,7 +438,7 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
         uint32_t r1 = L->atype_reqm[t1], r2 = L->atype_reqm[t2];
         bool cgg0 = (r1 == 24 && r2 == 25) || (r1 == 25 && r2 == 24);   // ATYPE_CG_IDX / ATYPE_G0_IDX
         bool fast = (m == 12) && (n == 6 || n == 10);
-        if (!fast) hd.any_general = 1;
+        if (!fast || (cgg0 && N > kFullPairAtoms)) hd.any_general = 1;
         ra.fn = (float)n;
         prx[q].flags = m | (n << 8) | (cgg0 ? kPairCgG0 : 0u) | (fast ? kPairFast : 0u);
         prx[q].atoms = (uint32_t)i | ((uint32_t)j << 16);
@@ -462,6 +463,13 @@ int build_ligand(adgpu_context* c, const adgpu_ligand* L, const adgpu_energy_par
         if (!(copies == 1 ? one : two)) continue;
         PairA* out = reinterpret_cast<PairA*>(blob.data() + hd.off_pair_a[copies - 1]);
         for (int q = 0; q < PP; q += 32) spread_slots(copies, slot_stride(N), prx + q, out + q);
+    }
+    if (N > kFullPairAtoms) {
+        static_assert(kFullPairAtoms >= kSlotCopyAtoms, "compact records name one copy's slots");
+        PairC* out = reinterpret_cast<PairC*>(blob.data() + hd.off_pair_c);
+        for (int q = 0; P && q < PP; ++q)
+            out[q] = PairC{pra[q].ij | (pra[q].fn == 10.0f ? kPairTen : 0u), pra[q].ac, pra[q].bd,
+                           prb[q].reqm, prb[q].cq, prb[q].dsol};
     }
     std::memcpy(blob.data(), &hd, sizeof(hd));
     return ADGPU_OK;

@@ -31,6 +31,23 @@ struct __attribute__((aligned(16))) PairB {
     float dsol;       // (S1 + qasp|q1|) V2 + (S2 + qasp|q2|) V1
     float g;          // CG-G0 bond constant G: 50 for a CG-G0 pair, else 0
 };
+// The same in 24 bytes, for kernels that take gradients of ligands of more than
+// kFullPairAtoms atoms: the exponent as a bit, the CG-G0 constant with the
+// pair's flags.  The pairs of 90 atoms then fit in LDS beside 16 wavefronts of
+// a compute unit, where in 32 bytes they are read from memory: FIRE nrun 20 84
+// -> 93 M evals/s, nrun 60 99 -> 105, ADADELTA nrun 40 197 -> 209, ADAM nrun 10
+// on 84 atoms 68 -> 69.7.  At 70 and 77 atoms both fit, and FIRE and ADAM take
+// the same time with either (155 / 145 M); Solis-Wets' shorter step pays for
+// the unpacking (77 atoms 130 -> 125 M), so energies keep 32 bytes, and so do
+// smaller ligands (30 atoms, ADADELTA nrun 20: 528 -> 519 M).
+struct __attribute__((aligned(8))) PairC {
+    uint32_t ij;      // as PairA, | kPairTen
+    float ac, bd, reqm, cq, dsol;
+};
+constexpr uint32_t kPairTen = 1u << 31;   // n = 10 (else 6, or what the flags hold)
+constexpr int kFullPairAtoms = 64;
+// Whether a kernel for ligands of up to max_atoms atoms reads PairC.
+__host__ __device__ constexpr bool compact_pairs(int max_atoms, bool grad) { return grad && max_atoms > kFullPairAtoms; }
 // What only rare paths read of a pair, in a third array.
 struct PairX {
     uint32_t flags;   // m | n << 8 | (CG-G0 bond) << 16 | (12-6 / 12-10 form) << 17
@@ -67,7 +84,7 @@ __host__ __device__ inline int padded_pairs(int pairs, int to) { return (pairs +
 // Offsets are in bytes from the start of the block.
 struct LigandDev {
     int32_t num_atoms, true_ligand_atoms, num_rotbonds, num_genes;
-    int32_t num_pairs, nchunk, any_general, pad1;   // any_general: some pair is not 12-6 / 12-10
+    int32_t num_pairs, nchunk, any_general, pad1;   // any_general: some pair needs its flags (not 12-6 / 12-10, or CG-G0)
     float coeff_elec, coeff_desolv, qasp, half_smooth;
     float elec_min_distance, inv_elec_min, pad3, pad4;
     uint32_t off_atom_ref;    // float4 [N]  x, y, z (grid units), charge
@@ -78,6 +95,7 @@ struct LigandDev {
     uint32_t off_tor_atoms;   // int2   [T]  bond atoms
     uint32_t off_pair_a[2];   // PairA[P padded to kPairPad] for one and for two slot copies
     uint32_t off_pair_b;      // PairB[P padded]
+    uint32_t off_pair_c;      // PairC[P padded], above kFullPairAtoms atoms (for one slot copy)
     uint32_t off_pair_x;      // PairX[P padded]
     uint32_t off_type_ds;     // float2 [num_atypes] (dspars_S, dspars_V) per ligand type (FP64 re-scoring)
     uint32_t total_bytes;

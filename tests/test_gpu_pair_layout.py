@@ -119,3 +119,38 @@ def test_adam_past_its_table(gpu_ctx, c1):
         last = d["ene"]
     gpu_ctx.ligand_release(lid)
     gpu_ctx.maps_release(mid)
+
+
+@pytest.mark.parametrize("atoms, torsions, width", [(65, 8, 64), (66, 8, 32), (90, 12, 64), (130, 12, 64)])
+def test_compact_pair_records(gpu_ctx, atoms, torsions, width):
+    """Gradient kernels read the pairs of more than 64 atoms in 24 bytes: energies
+    and gradients with both exponents, with others and with CG-G0 bonds, whose
+    terms the compact record leaves to the flags."""
+    case = helpers.synthetic_case(atoms, torsions, lig_seed=atoms, map_seed=4, npts=48)
+    exps = np.array(case.tables.vw_exp).copy()
+    ten = exps.copy()
+    ten[::2] = (12 << 8) + 10
+    exps[1::3] = (9 << 8) + 7
+    types = np.array(case.tables.atype_reqm).copy()
+    types[:2] = (24, 25)
+    mid = gpu_ctx.maps_upload(case.packed, case.size, case.maps.num_map_atypes, case.spacing)
+    gpu_ctx.set_team_width(width)
+    try:
+        for form in (case, _with(case, vw_exp=ten), _with(case, vw_exp=exps), _with(case, atype_reqm=types)):
+            lid = gpu_ctx.ligand_upload(form.tables, form.ep)
+            poses = helpers.poses_for(form, 60, seed=78)
+            e, g = gpu_ctx.eval_poses(mid, lid, poses, adgpu.EVAL_ENERGRAD)
+            helpers.check_energies(form.orc, poses, e, edge_share=0.05)
+            e2, _ = gpu_ctx.eval_poses(mid, lid, poses, adgpu.EVAL_ENERGY)
+            helpers.check_energies(form.orc, poses, e2, e_ref=e, edge_share=0.05)
+            well = [0, 1, 2] + list(range(6, form.ng))
+            quantum = np.array([helpers.gene_quantum(form, k) for k in range(form.ng)])
+            off = 0
+            for p, row in zip(poses, g):
+                _, go = form.orc.energrad32(p, True)
+                off += int((np.abs(row[:form.ng] - go)[well] > (1e-4 * np.abs(go) + 4 * quantum)[well]).sum())
+            assert off <= 0.002 * len(poses) * len(well)
+            gpu_ctx.ligand_release(lid)
+    finally:
+        gpu_ctx.set_team_width(0)
+        gpu_ctx.maps_release(mid)
