@@ -2,10 +2,10 @@
 // the kernel translation units k_*.hip; each instantiates its own kernels).
 //
 // Execution model (CDNA, 64-wide wavefronts):
-//   * a "team" of TW lanes (TW = 32 or 64) evaluates one individual, so a
-//     wavefront carries 64/TW individuals; a 256-thread workgroup stages the
-//     ligand tables (pair records, torsion vectors) into LDS once and every
-//     team of the workgroup shares them;
+//   * a "team" of TW lanes (TW = 16, 32 or 64) evaluates one individual, so a
+//     wavefront carries 64/TW individuals; a workgroup stages the ligand
+//     tables (pair records, torsion vectors) into LDS once and every team of
+//     the workgroup shares them;
 //   * team lane l owns atoms l, l+TW, ... (NC chunks) and walks each atom's
 //     own torsion chain, so pose -> coordinates needs no barrier (the
 //     reference's rotation list is a barrier per cycle, calcenergy.cl:232-275);
@@ -14,8 +14,8 @@
 //     evaluates the sine/cosine of its own angle once per evaluation;
 //   * pairs are strided over the team; pair forces go to per-atom int32
 //     fixed-point accumulators in LDS through ds_add (order independent);
-//   * energies, forces and torques are summed with DPP row reductions plus
-//     readlane, which leaves identical bits in every lane of the team;
+//   * energies, forces and torques are summed with DPP row reductions and row
+//     swaps or broadcasts, in one order whatever the lanes that need the sum;
 //   * local searches run as persistent kernels: a team that finishes its
 //     entity takes the next one from a global counter, so teams of one
 //     wavefront never wait for each other and uneven searches balance out.
@@ -32,7 +32,7 @@
 namespace adgpu {
 
 #define DEV __device__ __forceinline__
-// Workgroups of up to 1024 threads; at least 4 wavefronts per SIMD (<= 128 VGPRs)
+// Workgroups of up to 1024 threads (choose_ls_shape).
 // Waves per SIMD the register budget is sized for (4: at most 128 VGPRs).
 #ifndef ADGPU_WAVES_PER_EU
 #define ADGPU_WAVES_PER_EU 4

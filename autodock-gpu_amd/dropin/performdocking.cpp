@@ -111,7 +111,7 @@ void to_adgpu_ligand(const Liganddata& lig, const kernelconstant_interintra& ki,
 
 std::vector<int> get_gpu_pool() {
     // eight hardware queues per process (HIP's default is 4) before the HIP
-    // runtime starts, so the library runs each job in four run groups
+    // runtime starts, for the streams of a job's run groups beside others
     setenv("GPU_MAX_HW_QUEUES", "8", 0);
     int n = 0;
     if (adgpu_device_count(&n) != ADGPU_OK || n <= 0) {

@@ -66,7 +66,7 @@ TRAFFIC_BYTES_PER_LS_EVAL = {("f32", 100, 150, "ad"): 494.3}
 # the kernel's VALU issue rate, reported against the device's VALU issue rate
 # on independent FP32 FMA chains measured live (adgpu_measure_valu_rate).
 # Keyed by (maps, nrun, pop, ls).
-LS_INSTR_PER_EVAL = {("f32", 100, 150, "ad"): (892.9, 73.2)}
+LS_INSTR_PER_EVAL = {("f32", 100, 150, "ad"): (775.6, 77.4)}
 
 
 def parse():
@@ -90,8 +90,8 @@ def parse():
     ap.add_argument("--graph-block", type=int, default=0, choices=[0, 2, 4, 8],
                     help="generations per captured hipGraph (adgpu_set_graph_block; 0 = launched one by one)")
     # hardware queues of this process, set before the HIP runtime starts (HIP's
-    # default is 4): with 8 the library runs the job's runs in four groups on
-    # four streams, each on its own queue
+    # default is 4); the library runs the job's runs in four groups on streams
+    # that it has seen run side by side
     ap.add_argument("--hw-queues", type=int, default=8, choices=range(1, 33), metavar="1..32")
     ap.add_argument("--workload", default="lga", choices=["lga", "serve", "screen", "poses", "flexres"])
     ap.add_argument("--poses", type=int, default=100000)
@@ -774,10 +774,10 @@ def main():
                                    "per_cu_per_clock_at_2p4ghz": rate / (256 * 2.4e9),
                                    "source": "instructions per evaluation from dispatch counters, four run "
                                              "groups with regrouping (dispatches serialized); peak = FP32 FMA "
-                                             "chains measured live by adgpu_measure_valu_rate; frac above 1: the "
-                                             "overlapping launches issue this mix faster than the FMA loop (its "
-                                             "v_mov and DPP moves take a fraction of an FMA's issue slot)"}
-        out["roofline"]["note"] = "the launch is VALU-issue-bound (valu); HBM traffic is 0.17 of the " \
+                                             "chains measured live by adgpu_measure_valu_rate, whose scalar "
+                                             "operands halve their rate: instructions with vector operands issue "
+                                             "faster, so frac can exceed 1"}
+        out["roofline"]["note"] = "the launch is bound by instruction issue (valu); HBM traffic is 0.17 of the " \
                                   "algorithmic bytes (the map set stays in L2 and the Infinity Cache)"
     if not a.no_cpu_baseline:
         out["cpu_baseline"] = cpu_baseline(maps, tables, ep, a.cpu_evals)
