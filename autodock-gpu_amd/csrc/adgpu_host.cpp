@@ -861,6 +861,7 @@ int adgpu_rescore_f64(adgpu_ctx c, int map_id, int lig_id, const float* genotype
 // beside the kept ones; those that do not stay until the end, so that the next
 // falls elsewhere.  Some 0.1 ms a stream, once per context; the context is held.
 static int make_lanes(adgpu_context* c) {
+    if (int rc = stage_reserve(c, 0, kStageOpen)) return rc;   // none where a larger one could not be had
     c->lanes_made = true;
     hipStream_t spare[3 * kMaxLanes] = {};
     int spares = 0;
