@@ -302,7 +302,7 @@ template <class V>
 DEV V* at(V* p, uint32_t bytes) { return reinterpret_cast<V*>(reinterpret_cast<char*>(p) + bytes); }
 
 struct TeamView {             // private to one team
-    float* cx;                // [slot_array] atom coordinates (grid units), one
+    float* cx;                // [coord_array] atom coordinates (grid units), one
     float* cy;                //   array per axis: lanes reading different
     float* cz;                //   atoms hit different banks
     int* fx;                  // [slot_array] int32 fixed-point pair forces
@@ -337,6 +337,17 @@ __host__ __device__ constexpr int coord_copies(int TW, int NC, bool PL, bool GRA
 }
 __host__ __device__ constexpr int coord_array(int TW, int NC, bool PL, bool GRAD) {
     return PL && !GRAD ? TW * NC + 4 : slot_array(TW, NC);
+}
+// Slot that lanes without an atom write, behind the atoms of every copy and
+// named by no pair: in one copy's arrays the first spare word, in two copies'
+// a slot between the first copy of a ligand of `atoms` atoms and its second.
+__host__ __device__ constexpr int idle_slot(int TW, int NC, bool PL, bool GRAD, int atoms) {
+    return coord_copies(TW, NC, PL, GRAD) == 2 ? slot_stride(atoms) - 16 : TW * NC;
+}
+// Whether its last copy lies inside the arrays for the shape's largest ligand.
+__host__ __device__ constexpr bool idle_slot_fits(int TW, int NC, bool PL, bool GRAD) {
+    return idle_slot(TW, NC, PL, GRAD, TW * NC) + (coord_copies(TW, NC, PL, GRAD) - 1) * slot_stride(TW * NC) <
+           coord_array(TW, NC, PL, GRAD);
 }
 
 __host__ __device__ inline size_t team_bytes_for(int TW, int NC, int T, bool PL, bool GRAD) {
@@ -432,7 +443,10 @@ struct Atoms {
     uint32_t copy;            // bytes from there to its second copy
     bool valid[NC], ign[NC], lig[NC];
 
+    // PL, GRAD: the kernel's layout, as stage is told.
+    template <bool PL, bool GRAD>
     DEV void load(const LigandDev* L, const GridDev& G) {
+        static_assert(idle_slot_fits(TW, NC, PL, GRAD), "lanes without an atom write inside their team's arrays");
         const char* gb = reinterpret_cast<const char*>(L);
         const float4* ar = reinterpret_cast<const float4*>(gb + L->off_atom_ref);
         const int4* ai = reinterpret_cast<const int4*>(gb + L->off_atom_info);
@@ -444,8 +458,7 @@ struct Atoms {
         for (int k = 0; k < NC; ++k) {
             int a = tl + TW * k;
             valid[k] = a < L->num_atoms;
-            // without an atom: the first slot behind them, which no pair names
-            slot[k] = 4u * (uint32_t)(valid[k] ? a : slot_copies(TW, NC) == 2 ? stride - 16 : TW * NC);
+            slot[k] = 4u * (uint32_t)(valid[k] ? a : idle_slot(TW, NC, PL, GRAD, L->num_atoms));
             int aa = valid[k] ? a : 0;
             float4 r = ar[aa];
             int4 inf = ai[aa];
@@ -1181,7 +1194,7 @@ struct Launch {
     EvalCtx<TW, NC> X;                                                         \
     X.L = a.L;                                                                 \
     X.G = a.G;                                                                 \
-    X.A.load(a.L, a.G);   /* its loads run beside the staging's */              \
+    X.A.template load<PL, GRAD>(a.L, a.G);   /* its loads run beside the staging's */ \
     X.ls.load(a.L);                                                            \
     stage<TW, NC, PL, GRAD>(a.L, lds, X.sv, X.tv);                             \
     const int tl = TM::lane();                                                 \
