@@ -154,3 +154,20 @@ def test_records_at_the_edges_of_chunks_and_bins(gpu_ctx, c1g, nrun, pop):
         _same_record(rec, ref, c)
     _same_record(job.autostop_final(), orc.final(asf * 3, e, total), "final")
     job.destroy()
+
+
+@pytest.mark.parametrize("groups", [1, 2, 4])
+@pytest.mark.parametrize("as_frequency", [1, 5])
+def test_no_generations_enqueued_long_behind_the_stop(gpu_ctx, c1g, monkeypatch, as_frequency, groups):
+    """A search that a test ends launches no more than the 16 generations that
+    may be in flight, and the one whose end shows the stop, behind the last
+    real one of every run group."""
+    monkeypatch.setenv("ADGPU_RUN_GROUPS", str(groups))
+    job = _job(gpu_ctx, c1g, 40, 150, ls="ad")
+    job.initpop()
+    job.set_autostop(True, stopstd=2.0, as_frequency=as_frequency)
+    gens, _ = job.run()
+    assert job.autostop_final()["autostopped"] == 1
+    assert gens < job.sp.max_generations
+    assert job.kernel_time(1)[1] <= groups * (gens + 16 + 1)
+    job.destroy()
