@@ -51,6 +51,7 @@ constexpr int kMaxLanes = 4;
 
 struct adgpu_context {
     int device = 0;
+    std::atomic<int> users{1};       // the caller until it closes the context, and every job (context_drop)
     hipStream_t stream = nullptr;
     std::map<int, MapSet> maps;
     std::map<int, LigandSet> ligands;
@@ -113,6 +114,7 @@ struct adgpu_job {
     int map_id = 0, ligand_id = 0;
     bool counted = false;               // holds a use of its maps and ligand
     bool has_lanes = false;             // its groups run on the context's lanes
+    bool holds_ctx = false;             // counted in the context's users
     // capacities of the device buffers; a serving slot reuses them for the
     // next request and grows them only when a request needs more
     size_t cap_ne = 0, cap_ls = 0;
@@ -611,18 +613,34 @@ int adgpu_open(int device, adgpu_ctx* out) {
     return ADGPU_OK;
 }
 
+// A job may be destroyed after its context was closed: what its destruction
+// touches, its lanes among it, stays until the last of them is gone.
+static void context_hold(adgpu_job* j) {
+    j->ctx->users++;
+    j->holds_ctx = true;
+}
+static void context_drop(adgpu_context* c) {
+    if (--c->users > 0) return;
+    for (int k = 0; k < c->lanes; ++k) (void)hipStreamDestroy(c->lane[k]);
+    delete c;
+}
+
 int adgpu_close(adgpu_ctx c) {
     if (!c) return ADGPU_ERR_ARG;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
-    for (auto& kv : c->maps) (void)hipFree(kv.second.data);
-    for (auto& kv : c->ligands) (void)hipFree(kv.second.dev);
-    for (int k = 0; k < c->lanes; ++k) (void)hipStreamDestroy(c->lane[k]);
-    if (c->stage) (void)hipHostFree(c->stage);
-    for (hipEvent_t e : c->stage_ev)
-        if (e) (void)hipEventDestroy(e);
-    (void)hipStreamDestroy(c->stream);
-    delete c;
+    {
+        std::lock_guard<std::mutex> lk(c->mu);
+        for (auto& kv : c->maps) (void)hipFree(kv.second.data);
+        for (auto& kv : c->ligands) (void)hipFree(kv.second.dev);
+        c->maps.clear();
+        c->ligands.clear();
+        if (c->stage) (void)hipHostFree(c->stage);
+        for (hipEvent_t e : c->stage_ev)
+            if (e) (void)hipEventDestroy(e);
+        (void)hipStreamDestroy(c->stream);
+    }
+    context_drop(c);
     return ADGPU_OK;
 }
 
@@ -1130,6 +1148,7 @@ int adgpu_job_create(adgpu_ctx c, int map_id, int lig_id, const adgpu_search_par
         if (ls_workgroup(la, (int)std::min<int64_t>(searches, INT32_MAX), sp->ls_method) > kGroupThreads) ng = 2;
     }
     if (const char* e = std::getenv("ADGPU_RUN_GROUPS")) ng = std::atoi(e);
+    context_hold(j.get());
     rc = job_open(j.get());
     if (!rc) rc = job_set_groups(j.get(), ng, nrun);
     if (!rc)
@@ -1173,6 +1192,7 @@ int adgpu_job_destroy(adgpu_job_t j) {
     if (j->ev_origin) (void)hipEventDestroy(j->ev_origin);
     if (j->h_stop) (void)hipHostFree(j->h_stop);
     if (j->h_ring) (void)hipHostFree(j->h_ring);
+    if (j->holds_ctx) context_drop(j->ctx);
     delete j;
     return ADGPU_OK;
 }
@@ -2056,6 +2076,7 @@ int slot_open(adgpu_context* c, int run_groups, int sharers, adgpu_job** out) {
     j->own_lig = true;
     j->sharers = std::max(1, sharers);
     j->want_groups = std::max(1, std::min(run_groups, kMaxGroups));
+    context_hold(j.get());
     int rc = job_open(j.get());
     if (!rc) rc = job_set_groups(j.get(), run_groups, run_groups);
     if (rc) {

@@ -266,3 +266,31 @@ def test_jobs_share_a_contexts_lanes(gpu_ctx, c1):
         assert np.array_equal(d0["pop"], d1["pop"]) and np.array_equal(d0["ene"], d1["ene"])
     gpu_ctx.ligand_release(lid)
     gpu_ctx.maps_release(mid)
+
+
+@pytest.mark.parametrize("nrun", [4, 40])
+def test_jobs_outlive_their_context(gpu_ctx, c1, nrun):
+    """Jobs may be destroyed after their context was closed, in any order, also
+    those that run on streams the context made for them."""
+    ctx = adgpu.Context(0)
+    mid = ctx.maps_upload(c1.packed, c1.size, c1.maps.num_map_atypes, c1.spacing)
+    lid = ctx.ligand_upload(c1.tables, c1.ep)
+    sp = search_params(num_runs=nrun, pop_size=100, max_evals=3000, ls="ad", spacing=c1.spacing, max_iters=10)
+    init = O.initial_population((1,), nrun, 100, c1.maps.size_angstr, c1.spacing)
+    jobs = [ctx.job(mid, lid, sp, init, O.cmwc_uints((1,), nrun * 100 * 64)) for _ in range(3)]
+    for j in jobs:
+        j.initpop()
+        j.run()
+    jobs[1].destroy()
+    ctx.close()
+    jobs[0].destroy()
+    jobs[2].destroy()
+    # the device is as before
+    mid = gpu_ctx.maps_upload(c1.packed, c1.size, c1.maps.num_map_atypes, c1.spacing)
+    lid = gpu_ctx.ligand_upload(c1.tables, c1.ep)
+    job = gpu_ctx.job(mid, lid, sp, init, O.cmwc_uints((1,), nrun * 100 * 64))
+    job.initpop()
+    assert job.run()[0] > 0
+    job.destroy()
+    gpu_ctx.ligand_release(lid)
+    gpu_ctx.maps_release(mid)
