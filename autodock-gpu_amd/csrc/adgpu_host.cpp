@@ -878,9 +878,11 @@ int adgpu_rescore_f64(adgpu_ctx c, int map_id, int lig_id, const float* genotype
 // two.  So streams are made one by one and kept when they are seen to run
 // beside the kept ones; those that do not stay until the end, so that the next
 // falls elsewhere.  Some 0.1 ms a stream, once per context; the context is held.
-static int make_lanes(adgpu_context* c) {
-    if (int rc = stage_reserve(c, 0, kStageOpen)) return rc;   // none where a larger one could not be had
+// Streams or memory that cannot be had end the search: jobs then run on what
+// lanes there are, or on streams of their own.
+static void make_lanes(adgpu_context* c) {
     c->lanes_made = true;
+    if (stage_reserve(c, 0, kStageOpen)) return;   // none where a larger one could not be had
     hipStream_t spare[3 * kMaxLanes] = {};
     int spares = 0;
     hipError_t e = hipSuccess;
@@ -894,8 +896,7 @@ static int make_lanes(adgpu_context* c) {
         else spare[spares++] = s;
     }
     for (int k = 0; k < spares; ++k) (void)hipStreamDestroy(spare[k]);
-    HIPCHK(c, e);
-    return ADGPU_OK;
+    if (e != hipSuccess) (void)hipGetLastError();
 }
 
 // Run groups: streams and their per-generation events.
@@ -1135,8 +1136,7 @@ int adgpu_job_create(adgpu_ctx c, int map_id, int lig_id, const adgpu_search_par
     int ng = 2;
     const int64_t searches = (int64_t)nrun * std::max(1, to_dev(sp, num_genes).num_ls);
     const bool several = searches >= 2 * kGroupSearches || std::getenv("ADGPU_RUN_GROUPS");
-    if (several && !c->lanes_made)
-        if (int rc = make_lanes(c)) return rc;
+    if (several && !c->lanes_made) make_lanes(c);
     if (several && c->lanes > 1 && !c->lanes_taken.exchange(true)) {
         j->has_lanes = true;   // until the job is destroyed
         ng = c->lanes;

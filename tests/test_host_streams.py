@@ -1,0 +1,80 @@
+"""Streams of contexts and jobs, on the CPU: the library's host code runs on a
+HIP runtime without a device (fake_hip.cpp), whose streams share a few modelled
+hardware queues, and the queues of the launches are looked at."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+REPO = os.path.dirname(HERE)
+
+PRELUDE = r"""
+import ctypes as C, json, sys
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+fake.fake_kernel.restype = C.c_char_p
+fake.fake_host_limit.argtypes = [C.c_size_t]
+sys.path[:0] = [%r, %r, %r]
+import numpy as np
+import adgpu, helpers
+case = helpers.synthetic_case(20, 4, 3, 5, npts=16)
+
+def context():
+    ctx = adgpu.Context(0)
+    ctx.ids = (ctx.maps_upload(case.packed, case.size, case.maps.num_map_atypes, case.spacing),
+               ctx.ligand_upload(case.tables, case.ep))
+    return ctx
+
+def job(ctx, nrun=60, ls="fire"):
+    sp = adgpu.search_params(num_runs=nrun, pop_size=100, ls=ls, spacing=case.spacing)
+    return ctx.job(*ctx.ids, sp, np.zeros((nrun * 100, 64), np.float32), np.ones(nrun * 6400, np.uint32))
+
+def launched(call, kernel):
+    fake.fake_clear()
+    call()
+    return [k for k in range(fake.fake_launches()) if kernel in fake.fake_kernel(k).decode()]
+
+def queues(j):
+    "the queue of every run group's local search"
+    return [fake.fake_queue(k) for k in launched(lambda: j.run(1), "k_ls_")]
+
+def pose_queue(ctx):
+    call = lambda: ctx.eval_poses(*ctx.ids, np.zeros((1, 64), np.float32))
+    return fake.fake_queue(launched(call, "k_eval_poses")[0])
+""" % (os.path.join(REPO, "autodock-gpu_amd"), os.path.join(REPO, "oracle"), HERE)
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", os.path.join(HERE, "fake_hip.cpp"), "-o", lib],
+                   check=True)
+    return lib
+
+
+def run(fake, code, hw_queues=None, **env):
+    e = {k: v for k, v in os.environ.items() if not k.startswith("ADGPU_") or k == "ADGPU_LIBRARY"}
+    e.pop("GPU_MAX_HW_QUEUES", None)
+    if hw_queues:
+        e["GPU_MAX_HW_QUEUES"] = str(hw_queues)
+    r = subprocess.run([sys.executable, "-c", PRELUDE + code, fake], env=dict(e, **env), capture_output=True,
+                       text=True, timeout=120)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return json.loads(r.stdout.splitlines()[-1])
+
+
+def test_a_job_is_not_refused_for_want_of_lanes(fake):
+    """Two queues have no four streams apart; the search for them ends where no
+    more streams can be had, and gives its own back."""
+    got, alive = run(fake, """
+fake.fake_streams_limit(6)
+ctx = context()
+j = job(ctx)
+got = queues(j)
+j.destroy()
+ctx.close()
+print(json.dumps([got, fake.fake_streams_alive()]))
+""", 2)
+    assert len(got) == 2 and alive == 0
