@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -70,10 +71,10 @@ struct adgpu_context {
     size_t stage_bytes = 0;
     hipEvent_t stage_ev[kStageParts] = {};
     // streams that were seen to run side by side, for the run groups of one job
-    // at a time (make_lanes); more jobs at once make streams of their own
+    // at a time (find_lanes)
     hipStream_t lane[kMaxLanes] = {};
     int lanes = 0;
-    bool lanes_made = false;
+    int lanes_asked = 0, lanes_next = 1;   // jobs that found too few, and which of them looks again
     std::atomic<bool> lanes_taken{false};
     float* noalloc = nullptr;  // this device's staging area of adgpu_eval_poses_noalloc
 };
@@ -869,7 +870,14 @@ int adgpu_rescore_f64(adgpu_ctx c, int map_id, int lig_id, const float* genotype
     return ADGPU_OK;
 }
 
-// Makes the context's lanes: up to kMaxLanes streams on hardware queues of
+// Hardware queues that the runtime spreads a process's streams over.
+static int hardware_queues() {
+    const char* e = std::getenv("GPU_MAX_HW_QUEUES");
+    const int n = e ? std::atoi(e) : 0;
+    return n > 0 ? n : 4;   // HIP's default
+}
+
+// Looks for the context's lanes: up to kMaxLanes streams on hardware queues of
 // their own.  The runtime spreads a process's streams over its hardware
 // queues (GPU_MAX_HW_QUEUES, four unless set) by a rule of its own, and
 // kernels of streams that share a queue run one after the other: the docking
@@ -877,23 +885,35 @@ int adgpu_rescore_f64(adgpu_ctx c, int map_id, int lig_id, const float* genotype
 // contexts open and 600 ms with one, in two groups 385 and 600 ms with one and
 // two.  So streams are made one by one and kept when they are seen to run
 // beside the kept ones; those that do not stay until the end, so that the next
-// falls elsewhere.  Some 0.1 ms a stream, once per context; the context is held.
-// Streams or memory that cannot be had end the search: jobs then run on what
-// lanes there are, or on streams of their own.
-static void make_lanes(adgpu_context* c) {
-    c->lanes_made = true;
+// falls elsewhere: some 0.1 ms for a stream that stays, 2.5 for one that does
+// not (a second, longer look in case other work filled the device or the host
+// was held up).  What is missed all the same, or because a stream could not be
+// had, is looked for again by the 2nd, 4th, 8th ... job that needs it;
+// meanwhile jobs make streams of their own.  The context is held.
+static void find_lanes(adgpu_context* c) {
+    if (c->lanes >= kMaxLanes || c->lanes_taken || ++c->lanes_asked < c->lanes_next) return;
+    c->lanes_next = 2 * c->lanes_asked;
     if (stage_reserve(c, 0, kStageOpen)) return;   // none where a larger one could not be had
-    hipStream_t spare[3 * kMaxLanes] = {};
+    constexpr int kSpares = 3 * kMaxLanes;
+    constexpr std::chrono::milliseconds kBusy(20);
+    hipStream_t spare[kSpares] = {};
     int spares = 0;
     hipError_t e = hipSuccess;
-    while (c->lanes < kMaxLanes && spares < 3 * kMaxLanes && e == hipSuccess) {
+    std::chrono::steady_clock::time_point first{};
+    for (int k = 0; c->lanes < kMaxLanes && spares < kSpares && e == hipSuccess; ++k) {
         hipStream_t s = nullptr;
-        bool apart = false;
         e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
         if (e != hipSuccess) break;
-        e = streams_overlap(s, c->lane, c->lanes, reinterpret_cast<uint64_t*>(c->stage), &apart);
+        bool apart = false;
+        for (int us : {60, 2000}) {
+            if (apart || e != hipSuccess) break;
+            e = streams_overlap(s, c->lane, c->lanes, us, reinterpret_cast<uint64_t*>(c->stage), &apart);
+        }
         if (e == hipSuccess && apart) c->lane[c->lanes++] = s;
         else spare[spares++] = s;
+        const auto now = std::chrono::steady_clock::now();
+        if (k == 0) first = now;   // the first trial loads the kernels
+        else if (now - first > kBusy) break;
     }
     for (int k = 0; k < spares; ++k) (void)hipStreamDestroy(spare[k]);
     if (e != hipSuccess) (void)hipGetLastError();
@@ -1122,25 +1142,30 @@ int adgpu_job_create(adgpu_ctx c, int map_id, int lig_id, const adgpu_search_par
     j->ligand_id = lig_id;
     const int nrun = sp->num_runs;
     // run groups: ADGPU_RUN_GROUPS streams.  Groups whose streams share a
-    // hardware queue serialize, so there are as many as the context has lanes
-    // (four with the HIP runtime's four hardware queues or more), and two when
-    // another job has them.  A group's local-search launch should still fill a
-    // good part of the device, so small jobs get fewer groups: one per
-    // kGroupSearches searches of a generation.  Launches in workgroups above
-    // 256 threads (large pair lists) overlap worse: two groups.  ms a docking
-    // in 1 / 2 / 3 / 4 groups on four queues: FIRE nrun 20, 30 atoms 49 / 47 /
-    // 52 / 59; Solis-Wets nrun 50, 30 atoms 72 / 59 / 60 / 58; ADADELTA nrun
-    // 100, 23 atoms 64 / 57 / 57 / 52, 30 atoms - / 364 / 369 / 346; ADAM nrun
-    // 50, 41 atoms - / 116 / 116 / 111; ADADELTA nrun 50, 54 atoms (512
-    // threads) - / 186 / 195 / 191.
-    int ng = 2;
+    // hardware queue serialize, so there are four where as many lanes were
+    // found, or six queues make it likely that four streams fall apart, else
+    // two; and two beside a job that has the lanes (two dockings of 30 atoms,
+    // ADADELTA nrun 100, at once on eight queues: 640 ms, with four groups each
+    // 745).  A group's local-search launch should still fill a good part of
+    // the device, so small jobs get fewer groups: one per kGroupSearches
+    // searches of a generation.  Launches in workgroups above 256 threads (large
+    // pair lists) overlap worse: two groups.  ms a docking in 1 / 2 / 3 / 4 groups
+    // on streams apart: FIRE nrun 20, 30 atoms 25.8 / 24.4 / 27.2 / 31.4;
+    // Solis-Wets, 30 atoms, nrun 20 91.7 / 86.5 / 82.6 / 85.0, nrun 50 184.2 /
+    // 148.5 / 148.9 / 144.7; ADADELTA nrun 100, 23 atoms 340 / 289 / 286 /
+    // 280, 30 atoms 445 / 363 / 367 / 346; ADAM nrun 50, 41 atoms 122.1 /
+    // 113.4 / 112.8 / 109.2; in 512 threads ADADELTA nrun 50, 54 atoms 221.5 /
+    // 185.8 / 197.0 / 194.8, FIRE nrun 20, 90 atoms 123.4 / 123.2 / 145.2 /
+    // 126.9.
     const int64_t searches = (int64_t)nrun * std::max(1, to_dev(sp, num_genes).num_ls);
-    const bool several = searches >= 2 * kGroupSearches || std::getenv("ADGPU_RUN_GROUPS");
-    if (several && !c->lanes_made) make_lanes(c);
-    if (several && c->lanes > 1 && !c->lanes_taken.exchange(true)) {
-        j->has_lanes = true;   // until the job is destroyed
-        ng = c->lanes;
+    const int queues = hardware_queues();
+    bool lent = false;
+    if (searches >= 2 * kGroupSearches || std::getenv("ADGPU_RUN_GROUPS")) {
+        find_lanes(c);
+        lent = c->lanes > 1 && c->lanes_taken.exchange(true);
+        j->has_lanes = c->lanes > 1 && !lent;   // until the job is destroyed
     }
+    int ng = !lent && (c->lanes == kMaxLanes || queues >= 6) ? 4 : 2;
     ng = (int)std::max<int64_t>(1, std::min<int64_t>(ng, searches / kGroupSearches));
     if (ng > 2) {
         const int tw = job_team_width(c, li->second.host.num_atoms, searches, 1, sp->ls_method);

@@ -221,10 +221,10 @@ hipError_t noalloc_scratch_setup(int device, float** out);
 hipError_t eval_poses_noalloc(const LaunchArgs& la, float* scratch_dev, int mode, const float* genotypes, int n,
                               float* energies, float* grads);
 // Whether kernels of stream s run beside those of each of n other streams, none
-// of them in use: a kernel holds s for 60 us, and the others' must start
+// of them in use: a kernel holds s for hold_us, and the others' must start
 // before it ends.  span: 2 + 2 n pinned words.  False also where the host was
-// held up in between.
-hipError_t streams_overlap(hipStream_t s, const hipStream_t* others, int n, uint64_t* span, bool* all);
+// held up in between, or other work left no room for the others in that time.
+hipError_t streams_overlap(hipStream_t s, const hipStream_t* others, int n, int hold_us, uint64_t* span, bool* all);
 // Wavefront VALU instructions per second of a kernel of independent FP32
 // FMA chains over `blocks` workgroups of 256 threads (k_calib.hip); scratch
 // holds blocks * 256 floats.

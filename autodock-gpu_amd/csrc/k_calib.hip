@@ -46,11 +46,11 @@ __global__ __launch_bounds__(64) void k_hold(uint64_t* span, uint32_t ticks) {
 
 }  // namespace
 
-hipError_t streams_overlap(hipStream_t s, const hipStream_t* others, int n, uint64_t* span, bool* all) {
+hipError_t streams_overlap(hipStream_t s, const hipStream_t* others, int n, int hold_us, uint64_t* span, bool* all) {
     *all = false;
     // the first launch on a stream may wait for its queue: once before the test
     for (int round = 0; round < 2; ++round) {
-        hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, s, span, round ? 6000u : 10u);
+        hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, s, span, round ? 100u * (uint32_t)hold_us : 10u);
         for (int k = 0; k < n; ++k)
             hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, others[k], span + 2 + 2 * k, 10u);
         hipError_t e = hipGetLastError();

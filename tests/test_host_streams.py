@@ -65,6 +65,41 @@ def run(fake, code, hw_queues=None, **env):
     return json.loads(r.stdout.splitlines()[-1])
 
 
+def test_jobs_beside_one_that_has_the_lanes(fake):
+    """They run in two groups on streams of their own; the lanes go to the next
+    job after the first was destroyed."""
+    first, second, third = run(fake, """
+ctx = context()
+a = job(ctx); b = job(ctx)
+out = [queues(a), queues(b)]
+a.destroy()
+c = job(ctx)
+print(json.dumps(out + [queues(c)]))
+""", 8)
+    assert len(second) == 2
+    assert len(first) == len(third) == 4 and set(first) == set(third)
+
+
+def test_lanes_missed_on_a_busy_device_are_looked_for_again(fake):
+    """A first job that meets a busy device runs all the same, in as many groups
+    as the queues allow; a later one has lanes."""
+    first, later = run(fake, """
+ctx = context()
+fake.fake_busy(1)
+a = job(ctx)
+fake.fake_busy(0)
+out = [queues(a)]
+a.destroy()
+for _ in range(2):
+    b = job(ctx)
+    got = queues(b)
+    b.destroy()
+print(json.dumps(out + [got]))
+""", 8)
+    assert len(first) == 4
+    assert len(later) == 4 and len(set(later)) == 4
+
+
 def test_a_job_is_not_refused_for_want_of_lanes(fake):
     """Two queues have no four streams apart; the search for them ends where no
     more streams can be had, and gives its own back."""
@@ -78,3 +113,16 @@ ctx.close()
 print(json.dumps([got, fake.fake_streams_alive()]))
 """, 2)
     assert len(got) == 2 and alive == 0
+
+
+def test_searches_for_lanes_become_rare(fake):
+    """Where there are no lanes to be found, 32 jobs look for them 6 times."""
+    got = run(fake, """
+ctx = context()
+n = 0
+for _ in range(32):
+    hold = launched(lambda: job(ctx).destroy(), "k_hold")
+    n += bool(hold)
+print(json.dumps(n))
+""", 1)
+    assert got == 6
