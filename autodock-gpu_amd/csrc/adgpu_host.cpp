@@ -70,8 +70,8 @@ struct adgpu_context {
     char* stage = nullptr;
     size_t stage_bytes = 0;
     hipEvent_t stage_ev[kStageParts] = {};
-    // streams that were seen to run side by side, for the run groups of one job
-    // at a time (find_lanes)
+    // streams that were seen to run beside each other and beside `stream`, for
+    // the run groups of one job at a time (find_lanes)
     hipStream_t lane[kMaxLanes] = {};
     int lanes = 0;
     int lanes_asked = 0, lanes_next = 1;   // jobs that found too few, and which of them looks again
@@ -877,21 +877,24 @@ static int hardware_queues() {
     return n > 0 ? n : 4;   // HIP's default
 }
 
-// Looks for the context's lanes: up to kMaxLanes streams on hardware queues of
-// their own.  The runtime spreads a process's streams over its hardware
-// queues (GPU_MAX_HW_QUEUES, four unless set) by a rule of its own, and
-// kernels of streams that share a queue run one after the other: the docking
-// of 30 atoms, ADADELTA nrun 100, took 345 ms in four groups with three
-// contexts open and 600 ms with one, in two groups 385 and 600 ms with one and
-// two.  So streams are made one by one and kept when they are seen to run
-// beside the kept ones; those that do not stay until the end, so that the next
-// falls elsewhere: some 0.1 ms for a stream that stays, 2.5 for one that does
-// not (a second, longer look in case other work filled the device or the host
-// was held up).  What is missed all the same, or because a stream could not be
+// Looks for the context's lanes: `want` streams on hardware queues of their
+// own, apart from each other and from the context's stream.  The runtime
+// spreads streams over its queues by a rule of its own, and kernels of streams
+// that share a queue run one after the other: the docking of 30 atoms,
+// ADADELTA nrun 100, took 345 ms in four groups with three contexts open and
+// 600 ms with one, in two groups 385 and 600 ms with one and two; and a pose
+// call of the context waits for all that a job has enqueued on its queue (one
+// pose beside that docking, four queues: 24 us and at most 1.6 ms, but 7 ms on
+// average and up to 58 with a lane on every queue).
+// So streams are made one by one and kept when they are seen to run beside the
+// kept ones; those that do not stay until the end, so that the next falls
+// elsewhere: some 0.1 ms for a stream that stays, 2.5 for one that does not
+// (a second, longer look in case other work filled the device or the host was
+// held up).  What is missed all the same, or because a stream could not be
 // had, is looked for again by the 2nd, 4th, 8th ... job that needs it;
 // meanwhile jobs make streams of their own.  The context is held.
-static void find_lanes(adgpu_context* c) {
-    if (c->lanes >= kMaxLanes || c->lanes_taken || ++c->lanes_asked < c->lanes_next) return;
+static void find_lanes(adgpu_context* c, int want) {
+    if (c->lanes >= want || c->lanes_taken || ++c->lanes_asked < c->lanes_next) return;
     c->lanes_next = 2 * c->lanes_asked;
     if (stage_reserve(c, 0, kStageOpen)) return;   // none where a larger one could not be had
     constexpr int kSpares = 3 * kMaxLanes;
@@ -900,14 +903,16 @@ static void find_lanes(adgpu_context* c) {
     int spares = 0;
     hipError_t e = hipSuccess;
     std::chrono::steady_clock::time_point first{};
-    for (int k = 0; c->lanes < kMaxLanes && spares < kSpares && e == hipSuccess; ++k) {
+    for (int k = 0; c->lanes < want && spares < kSpares && e == hipSuccess; ++k) {
         hipStream_t s = nullptr;
         e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
         if (e != hipSuccess) break;
+        hipStream_t others[kMaxLanes + 1] = {c->stream};
+        std::copy(c->lane, c->lane + c->lanes, others + 1);
         bool apart = false;
         for (int us : {60, 2000}) {
             if (apart || e != hipSuccess) break;
-            e = streams_overlap(s, c->lane, c->lanes, us, reinterpret_cast<uint64_t*>(c->stage), &apart);
+            e = streams_overlap(s, others, c->lanes + 1, us, reinterpret_cast<uint64_t*>(c->stage), &apart);
         }
         if (e == hipSuccess && apart) c->lane[c->lanes++] = s;
         else spare[spares++] = s;
@@ -1161,7 +1166,7 @@ int adgpu_job_create(adgpu_ctx c, int map_id, int lig_id, const adgpu_search_par
     const int queues = hardware_queues();
     bool lent = false;
     if (searches >= 2 * kGroupSearches || std::getenv("ADGPU_RUN_GROUPS")) {
-        find_lanes(c);
+        find_lanes(c, queues > kMaxLanes ? kMaxLanes : 2);
         lent = c->lanes > 1 && c->lanes_taken.exchange(true);
         j->has_lanes = c->lanes > 1 && !lent;   // until the job is destroyed
     }

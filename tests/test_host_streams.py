@@ -65,6 +65,21 @@ def run(fake, code, hw_queues=None, **env):
     return json.loads(r.stdout.splitlines()[-1])
 
 
+@pytest.mark.parametrize("hw_queues, groups", [(None, 2), (3, 2), (4, 2), (5, 4), (8, 4)])
+@pytest.mark.parametrize("others", [0, 1, 3])
+def test_groups_run_apart_and_leave_the_contexts_queue(fake, hw_queues, groups, others):
+    """A job's groups have a queue each, and none has that of the context's
+    pose calls, however many other contexts took streams before."""
+    got = run(fake, """
+more = [context() for _ in range(%d)]
+ctx = context()
+j = job(ctx)
+print(json.dumps([queues(j), pose_queue(ctx)]))
+""" % others, hw_queues)
+    assert len(got[0]) == groups
+    assert len(set(got[0] + [got[1]])) == groups + 1, got
+
+
 def test_jobs_beside_one_that_has_the_lanes(fake):
     """They run in two groups on streams of their own; the lanes go to the next
     job after the first was destroyed."""
