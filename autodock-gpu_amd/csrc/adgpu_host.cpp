@@ -602,10 +602,8 @@ int adgpu_open(int device, adgpu_ctx* out) {
         (void)hipStreamDestroy(c->stream);
         return ADGPU_ERR_HIP;
     }
-    if (stage_reserve(c.get(), 0, kStageOpen) != ADGPU_OK) {
-        (void)hipStreamDestroy(c->stream);
-        return ADGPU_ERR_NOMEM;
-    }
+    // ahead of the first pose call; where it cannot be had now, the call asks again
+    (void)stage_reserve(c.get(), 0, kStageOpen);
     if (const char* tw = std::getenv("ADGPU_TEAM_WIDTH")) {
         int v = std::atoi(tw);
         c->team_hint = (v == 16 || v == 32 || v == 64) ? v : 0;

@@ -1,6 +1,6 @@
-"""Streams of contexts and jobs, on the CPU: the library's host code runs on a
-HIP runtime without a device (fake_hip.cpp), whose streams share a few modelled
-hardware queues, and the queues of the launches are looked at."""
+"""Streams and launches of contexts and jobs, on the CPU: the library's host
+code runs on a HIP runtime without a device (fake_hip.cpp), whose streams share
+a few modelled hardware queues and whose memory and streams can be bounded."""
 import json
 import os
 import subprocess
@@ -141,3 +141,24 @@ for _ in range(32):
 print(json.dumps(n))
 """, 1)
     assert got == 6
+
+
+def test_a_context_opens_without_pinned_memory(fake):
+    """Uploads and jobs need no staging memory; a pose call says that it could
+    not be had, and asks again the next time."""
+    refused, groups, energies = run(fake, """
+fake.fake_host_limit(4096)
+ctx = context()
+try:
+    ctx.eval_poses(*ctx.ids, np.zeros((1, 64), np.float32))
+    refused = ""
+except adgpu.AdgpuError as e:
+    refused = str(e)
+j = job(ctx)
+groups = len(queues(j))
+j.destroy()
+fake.fake_host_limit(1 << 40)
+e, _ = ctx.eval_poses(*ctx.ids, np.zeros((5, 64), np.float32))
+print(json.dumps([refused, groups, len(e)]))
+""", 4)
+    assert "pose staging" in refused and groups == 2 and energies == 5
