@@ -1275,11 +1275,12 @@ inline Shape choose_shape(const LigandDev& L, int team_width_hint, bool grad, in
 // FIRE, nrun 60 185 against 147, Solis-Wets 165 against 127.  A server's
 // launches keep 256 threads: larger workgroups need half or all of a compute
 // unit free at once, which the launches of other requests seldom leave (24
-// ligands in 16 slots 0.56 s against 0.50 s).
-inline Shape choose_ls_shape(const LaunchArgs& la, int searches, bool grad, int threads) {
+// ligands in 16 slots 0.56 s against 0.50 s).  fixed: the threads if they are
+// not to be chosen, else 0.
+inline Shape choose_ls_shape(const LaunchArgs& la, int searches, bool grad, int fixed) {
     const LigandDev& L = *la.lig_host;
-    Shape s = choose_shape(L, la.team_hint, grad, threads);
-    if (la.crowded || threads != kGroupThreads) return s;
+    Shape s = choose_shape(L, la.team_hint, grad, fixed ? fixed : kGroupThreads);
+    if (la.crowded || fixed) return s;
     // wavefronts of all the launches that share the device, were they like this one
     const int64_t need = ((int64_t)searches * s.tw + kWave - 1) / kWave * la.share;
     int64_t best = INT64_MIN;

@@ -36,13 +36,15 @@ inline int resident_groups(const void* kfn, size_t lds, int threads = 256) {
     return n;
 }
 
-// Workgroup size of the persistent local-search launches: smaller groups
-// release their compute-unit slots sooner when a launch drains, so another
-// run group's launch can move in.  ADGPU_LS_BLOCK = 64, 128 or 256.
+// Workgroup size that ADGPU_LS_BLOCK fixes for the persistent local-search
+// launches (64, 128, else 256), 0 where it is not set.  Smaller groups release
+// their compute-unit slots sooner when a launch drains, so another run group's
+// launch can move in.
 inline int ls_group_threads() {
     static const int t = [] {
         const char* e = std::getenv("ADGPU_LS_BLOCK");
-        const int v = e ? std::atoi(e) : 256;
+        if (!e) return 0;
+        const int v = std::atoi(e);
         return (v == 64 || v == 128) ? v : 256;
     }();
     return t;

@@ -163,7 +163,7 @@ hipError_t launch_ls_fire(const LaunchArgs& la, const SearchDev& sp, const JobBu
         err = hipGetLastError();
     });
     if (err != hipSuccess) return err;
-    // the persistent loop, in workgroups of ls_group_threads()
+    // the persistent loop, in workgroups of a size of its own
     const Shape shl = choose_ls_shape(la, n, true, ls_group_threads());
     const int want_l = (n + shl.threads / shl.tw - 1) / (shl.threads / shl.tw);
     ADGPU_DISPATCH(k_ls_fire, shl, la.grid.format, {

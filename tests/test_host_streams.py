@@ -162,3 +162,26 @@ e, _ = ctx.eval_poses(*ctx.ids, np.zeros((5, 64), np.float32))
 print(json.dumps([refused, groups, len(e)]))
 """, 4)
     assert "pose staging" in refused and groups == 2 and energies == 5
+
+
+WORKGROUPS = """
+ctx = context()
+def threads(atoms, torsions, width, nrun, ls):
+    c = helpers.synthetic_case(atoms, torsions, lig_seed=atoms, map_seed=4, npts=16)
+    ctx.set_team_width(width)
+    ids = ctx.maps_upload(c.packed, c.size, c.maps.num_map_atypes, c.spacing), ctx.ligand_upload(c.tables, c.ep)
+    sp = adgpu.search_params(num_runs=nrun, pop_size=150, ls=ls, spacing=c.spacing)
+    j = ctx.job(*ids, sp, np.zeros((nrun * 150, 64), np.float32), np.ones(nrun * 9600, np.uint32))
+    (k,) = launched(j.kernel_ls, "k_ls_")
+    return fake.fake_block(k)
+"""
+
+
+@pytest.mark.parametrize("block, threads", [("64", 64), ("128", 128), ("256", 256), ("512", 256)])
+def test_a_fixed_workgroup_size_is_kept(fake, block, threads):
+    """Also where launches in workgroups of more threads would hold the pair
+    records that 256 threads leave in memory."""
+    got = run(fake, WORKGROUPS + """
+print(json.dumps([threads(72, 10, 64, 40, ls) for ls in ("sw", "ad", "adam", "fire")]))
+""", ADGPU_LS_BLOCK=block)
+    assert got == [threads] * 4
