@@ -143,7 +143,7 @@ struct adgpu_job {
     int32_t* evals_runs = nullptr;
     uint32_t* prng = nullptr;
     int32_t* counters = nullptr;        // one LS work-queue counter per group (16 ints apart)
-    float2* adam_pow = nullptr;         // ADAM's bias corrections (kAdamPow entries)
+    float2* adam_pow = nullptr;         // ADAM's bias corrections (kAdamPow entries), from the first ADAM search
     int32_t* ls_ent = nullptr;
     float* ls_grad = nullptr;
     float* ls_state = nullptr;          // ADADELTA hand-off: saved searches, ring (cap_yield LS slots)
@@ -980,7 +980,6 @@ static int job_set_groups(adgpu_job* j, int ng, int nrun) {
 // Allocations of a job that do not depend on the request's size.
 static int job_open(adgpu_job* j) {
     bool ok = hipMalloc(&j->counters, 16 * kMaxGroups * sizeof(int32_t)) == hipSuccess &&
-              hipMalloc(&j->adam_pow, kAdamPow * sizeof(float2)) == hipSuccess &&
               hipMalloc(&j->d_stop, 16 * sizeof(int32_t)) == hipSuccess &&
               hipHostMalloc(&j->h_stop, 16 * sizeof(int32_t)) == hipSuccess &&
               hipEventCreateWithFlags(&j->ev_test, g_wait_event_flags.load()) == hipSuccess &&
@@ -1108,6 +1107,9 @@ static int job_start(adgpu_job* j, const adgpu_search_params* sp, const LigandDe
     j->spans[1].clear();
     j->kernel_ms[0] = j->kernel_ms[1] = 0.0;
     j->kernel_n[0] = j->kernel_n[1] = 0;
+    if (sp->ls_method == ADGPU_LS_ADAM && !j->adam_pow &&
+        hipMalloc(&j->adam_pow, kAdamPow * sizeof(float2)) != hipSuccess)
+        return fail(c, ADGPU_ERR_NOMEM, "job allocation failed");
     hipStream_t s = j->groups[0].stream;
     HIPCHK(c, hipMemcpyAsync(j->pop[0], init_pop, ne * kGenes * sizeof(float), hipMemcpyHostToDevice, s));
     HIPCHK(c, hipMemcpyAsync(j->pop[1], init_pop, ne * kGenes * sizeof(float), hipMemcpyHostToDevice, s));

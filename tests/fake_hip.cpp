@@ -22,6 +22,7 @@ struct Launch { std::string kernel; uint32_t grid, block; size_t lds; int stream
 std::recursive_mutex mu;
 int queues = 4, streams_made = 0, streams_alive = 0, streams_limit = 1 << 30, busy = 0;
 size_t host_limit = SIZE_MAX;
+std::vector<size_t> allocations;   // of device memory, in bytes
 std::vector<int> users;
 std::vector<uint64_t> queue_free;
 uint64_t now = 1;
@@ -48,7 +49,12 @@ void fake_streams_limit(int n) { streams_limit = n; }
 void fake_busy(int on) { busy = on; }
 void fake_host_limit(size_t bytes) { host_limit = bytes; }
 int fake_streams_alive() { return streams_alive; }
-void fake_clear() { launches.clear(); }
+void fake_clear() { launches.clear(); allocations.clear(); }
+int fake_allocations_of(size_t bytes) {
+    int n = 0;
+    for (size_t a : allocations) n += a == bytes;
+    return n;
+}
 int fake_launches() { return (int)launches.size(); }
 const char* fake_kernel(int i) { return launches[i].kernel.c_str(); }
 int fake_block(int i) { return (int)launches[i].block; }
@@ -133,11 +139,17 @@ int hipEventSynchronize(void*) { return 0; }
 int hipEventElapsedTime(float* ms, void*, void*) { *ms = 0.f; return 0; }
 
 // memory
-int hipMalloc(void** p, size_t n) { *p = std::calloc(n ? n : 1, 1); return *p ? 0 : 2; }
+int hipMalloc(void** p, size_t n) {
+    std::lock_guard<std::recursive_mutex> l(mu);
+    allocations.push_back(n);
+    *p = std::calloc(n ? n : 1, 1);
+    return *p ? 0 : 2;
+}
 int hipFree(void* p) { std::free(p); return 0; }
 int hipHostMalloc(void** p, size_t n, unsigned) {
     if (n > host_limit) { *p = nullptr; return 2; }
-    return hipMalloc(p, n);
+    *p = std::calloc(n ? n : 1, 1);
+    return *p ? 0 : 2;
 }
 int hipHostFree(void* p) { std::free(p); return 0; }
 int hipMemcpy(void* d, const void* s, size_t n, int) { std::memcpy(d, s, n); return 0; }

@@ -15,7 +15,7 @@ PRELUDE = r"""
 import ctypes as C, json, sys
 fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 fake.fake_kernel.restype = C.c_char_p
-fake.fake_host_limit.argtypes = [C.c_size_t]
+fake.fake_host_limit.argtypes = fake.fake_allocations_of.argtypes = [C.c_size_t]
 sys.path[:0] = [%r, %r, %r]
 import numpy as np
 import adgpu, helpers
@@ -185,3 +185,16 @@ def test_a_fixed_workgroup_size_is_kept(fake, block, threads):
 print(json.dumps([threads(72, 10, 64, 40, ls) for ls in ("sw", "ad", "adam", "fire")]))
 """, ADGPU_LS_BLOCK=block)
     assert got == [threads] * 4
+
+
+def test_only_adam_jobs_take_its_table(fake):
+    got = run(fake, """
+ctx = context()
+out = []
+for ls in ("sw", "ad", "fire", "adam"):
+    fake.fake_clear()
+    job(ctx, 3, ls).destroy()
+    out.append(fake.fake_allocations_of(8 * 1024))   # 1024 pairs of floats
+print(json.dumps(out))
+""")
+    assert got == [0, 0, 0, 1]
