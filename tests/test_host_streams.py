@@ -187,6 +187,24 @@ print(json.dumps([threads(72, 10, 64, 40, ls) for ls in ("sw", "ad", "adam", "fi
     assert got == [threads] * 4
 
 
+# atoms, torsions, team width, local search, runs of 150 searches, and the
+# threads of the workgroups that a launch of all their searches takes
+LARGE = [(54, 8, 32, "adam", 80, 512), (66, 10, 32, "sw", 80, 512), (80, 12, 32, "adam", 20, 512),
+         (80, 12, 32, "fire", 40, 768), (66, 10, 32, "ad", 80, 1024), (80, 12, 32, "sw", 80, 1024),
+         (60, 10, 64, "sw", 40, 512), (64, 10, 64, "ad", 20, 768), (84, 12, 64, "sw", 20, 768),
+         (64, 10, 64, "adam", 40, 1024), (84, 12, 64, "fire", 40, 1024), (84, 12, 64, "sw", 40, 1024)]
+
+
+def test_workgroup_sizes(fake):
+    """Larger workgroups than 256 threads are launched where they are meant to
+    be: for 32- and 64-lane teams, with and without gradients; two runs of the
+    same ligands take 256."""
+    got = run(fake, WORKGROUPS + """
+print(json.dumps([[threads(*c[:3], n, c[3]) for n in (c[4], 2)] for c in %r]))
+""" % (LARGE,))
+    assert got == [[c[5], 256] for c in LARGE]
+
+
 def test_only_adam_jobs_take_its_table(fake):
     got = run(fake, """
 ctx = context()
