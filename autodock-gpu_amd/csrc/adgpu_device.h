@@ -1275,9 +1275,15 @@ inline Shape choose_shape(const LigandDev& L, int team_width_hint, bool grad, in
 // FIRE, nrun 60 185 against 147, Solis-Wets 165 against 127.  A server's
 // launches keep 256 threads: larger workgroups need half or all of a compute
 // unit free at once, which the launches of other requests seldom leave (24
-// ligands in 16 slots 0.56 s against 0.50 s).  fixed: the threads if they are
-// not to be chosen, else 0.
-inline Shape choose_ls_shape(const LaunchArgs& la, int searches, bool grad, int fixed) {
+// ligands in 16 slots 0.56 s against 0.50 s).  So do ADADELTA's (uneven) where
+// others would take more than 512 or read PairC: a workgroup keeps its place
+// until its last search ends, and ADADELTA's differ in length by ten times.  M
+// evals/s in 256 threads against that: 60 atoms, nrun 50 / 100 147 / 202
+// against 132 / 182; 72 atoms, nrun 50 145 against 131; 90 atoms, nrun 40 / 100
+// 49 / 91 against 42 / 73.  (In 512 threads 54 atoms ran 221 against 230 at
+// nrun 50, 288 against 269 at nrun 100 and, on 126^3 maps, 283 against 260.)
+// fixed: the threads if they are not to be chosen, else 0.
+inline Shape choose_ls_shape(const LaunchArgs& la, int searches, bool grad, int fixed, bool uneven = false) {
     const LigandDev& L = *la.lig_host;
     Shape s = choose_shape(L, la.team_hint, grad, fixed ? fixed : kGroupThreads);
     if (la.crowded || fixed) return s;
@@ -1289,7 +1295,7 @@ inline Shape choose_ls_shape(const LaunchArgs& la, int searches, bool grad, int 
         const int w = t / kWave, fit = groups_per_cu(lds, t);
         const int64_t groups = (need + w - 1) / w;
         const bool all = groups <= (int64_t)fit * kCus;
-        if (!all && fit * w < 12) continue;
+        if (!all && (fit * w < 12 || (uneven && (t > 2 * kGroupThreads || compact_pairs(s.tw * s.nc, grad))))) continue;
         // all at once: prefer few wavefronts on the fullest compute unit; else many in all
         const int64_t score = all ? 2 * kCuWaves - (groups + kCus - 1) / kCus * w : fit * w - kCuWaves;
         if (score > best) {

@@ -110,7 +110,7 @@ hipError_t launch_sum_evals(hipStream_t s, const SearchDev& sp, const JobBuffers
 }
 
 int ls_workgroup(const LaunchArgs& la, int searches, int method) {
-    return choose_ls_shape(la, searches, method != ADGPU_LS_SW, ls_group_threads()).threads;
+    return choose_ls_shape(la, searches, method != ADGPU_LS_SW, ls_group_threads(), method == ADGPU_LS_AD).threads;
 }
 
 hipError_t launch_ls(const LaunchArgs& la, const SearchDev& sp, const JobBuffers& b, int method) {

@@ -333,7 +333,7 @@ hipError_t launch_ls_ad(const LaunchArgs& la, const SearchDev& sp, const JobBuff
     const int n = sp.num_runs * sp.num_ls;
     Launch a{};
     a.L = la.lig_dev; a.G = la.grid; a.S = sp; a.B = b;
-    const Shape sh = choose_ls_shape(la, n, true, ls_group_threads());
+    const Shape sh = choose_ls_shape(la, n, true, ls_group_threads(), true);
     const int per_group = sh.threads / sh.tw;
     hipError_t err = hipSuccess;
     ADGPU_DISPATCH(k_ls_ad, sh, la.grid.format, {

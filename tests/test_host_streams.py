@@ -190,8 +190,8 @@ print(json.dumps([threads(72, 10, 64, 40, ls) for ls in ("sw", "ad", "adam", "fi
 # atoms, torsions, team width, local search, runs of 150 searches, and the
 # threads of the workgroups that a launch of all their searches takes
 LARGE = [(54, 8, 32, "adam", 80, 512), (66, 10, 32, "sw", 80, 512), (80, 12, 32, "adam", 20, 512),
-         (80, 12, 32, "fire", 40, 768), (66, 10, 32, "ad", 80, 1024), (80, 12, 32, "sw", 80, 1024),
-         (60, 10, 64, "sw", 40, 512), (64, 10, 64, "ad", 20, 768), (84, 12, 64, "sw", 20, 768),
+         (80, 12, 32, "fire", 40, 768), (66, 10, 32, "adam", 80, 1024), (80, 12, 32, "sw", 80, 1024),
+         (60, 10, 64, "sw", 40, 512), (54, 8, 64, "ad", 80, 512), (64, 10, 64, "ad", 20, 768), (84, 12, 64, "sw", 20, 768),
          (64, 10, 64, "adam", 40, 1024), (84, 12, 64, "fire", 40, 1024), (84, 12, 64, "sw", 40, 1024)]
 
 
@@ -203,6 +203,16 @@ def test_workgroup_sizes(fake):
 print(json.dumps([[threads(*c[:3], n, c[3]) for n in (c[4], 2)] for c in %r]))
 """ % (LARGE,))
     assert got == [[c[5], 256] for c in LARGE]
+
+
+@pytest.mark.parametrize("atoms, width", [(64, 64), (66, 64), (84, 64), (80, 32)])
+def test_many_uneven_searches_stay_in_small_workgroups(fake, atoms, width):
+    """ADADELTA launches that do not hold all their searches at once, where
+    ADAM's take 512 to 1024 threads."""
+    ad, adam = run(fake, WORKGROUPS + """
+print(json.dumps([threads(%d, 10, %d, 80, ls) for ls in ("ad", "adam")]))
+""" % (atoms, width))
+    assert ad == 256 and adam >= 512
 
 
 def test_only_adam_jobs_take_its_table(fake):
