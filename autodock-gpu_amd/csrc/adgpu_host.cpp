@@ -738,7 +738,8 @@ int adgpu_ligand_release(adgpu_ctx c, int id) {
 // are packed and spread by up to four threads, a part each, while other parts
 // are on the device.  1 pose 31 -> 20 us; 4999 energies of 41 atoms 106 -> 55
 // us; energies and gradients of 1e5 poses of 30 atoms (25.6 MB in and out)
-// 3.0 -> 1.15 ms.  FP64 re-scoring of 100 poses 47 -> 32 us (24 with the kernel of today).
+// 3.0 -> 1.15 ms.  FP64 re-scoring of 100 poses 47 -> 32 us, and 24 with k_rescore_f64 in
+// 256 threads a pose.
 int adgpu_eval_poses(adgpu_ctx c, int map_id, int lig_id, int mode, const float* genotypes, int n,
                      float* energies, float* grads) {
     if (!c || !genotypes || n < 0) return fail(c, ADGPU_ERR_ARG, "null argument");

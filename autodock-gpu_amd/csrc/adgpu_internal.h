@@ -34,12 +34,14 @@ struct __attribute__((aligned(16))) PairB {
 // The same in 24 bytes, for kernels that take gradients of ligands of more than
 // kFullPairAtoms atoms: the exponent as a bit, the CG-G0 constant with the
 // pair's flags.  The pairs of 90 atoms then fit in LDS beside 16 wavefronts of
-// a compute unit, where in 32 bytes they are read from memory: FIRE nrun 20 84
-// -> 93 M evals/s, nrun 60 99 -> 105, ADADELTA nrun 40 197 -> 209, ADAM nrun 10
-// on 84 atoms 68 -> 69.7.  At 70 and 77 atoms both fit, and FIRE and ADAM take
-// the same time with either (155 / 145 M); Solis-Wets' shorter step pays for
-// the unpacking (77 atoms 130 -> 125 M), so energies keep 32 bytes, and so do
-// smaller ligands (30 atoms, ADADELTA nrun 20: 528 -> 519 M).
+// a compute unit, where in 32 bytes they are read from memory: dockings with
+// FIRE nrun 20 81.0 -> 89.7 M evals/s, nrun 60 96.3 -> 98.6, ADAM nrun 10 on 84
+// atoms 67.8 -> 68.7; ADADELTA's, in 256 threads, which read them from memory
+// in either form, nrun 40 48.4 -> 49.4 (100 atoms nrun 100 70.7 -> 72.2).  At 70
+// and 77 atoms both fit, and FIRE and ADAM take the same time with either
+// (137 / 132 M); Solis-Wets' shorter step pays for the unpacking (launches of
+// 77 atoms 130 -> 125 M), so energies keep 32 bytes, and so do smaller ligands
+// (30 atoms, ADADELTA nrun 20: 528 -> 519 M).
 struct __attribute__((aligned(8))) PairC {
     uint32_t ij;      // as PairA, | kPairTen
     float ac, bd, reqm, cq, dsol;
