@@ -53,9 +53,12 @@ hipError_t streams_overlap(hipStream_t s, const hipStream_t* others, int n, int 
         hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, s, span, round ? 100u * (uint32_t)hold_us : 10u);
         for (int k = 0; k < n; ++k)
             hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, others[k], span + 2 + 2 * k, 10u);
+        // whatever failed, none of them may be left to write to span later
         hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        for (int k = 0; k < n && e == hipSuccess; ++k) e = hipStreamSynchronize(others[k]);
+        for (int k = -1; k < n; ++k) {
+            const hipError_t w = hipStreamSynchronize(k < 0 ? s : others[k]);
+            if (e == hipSuccess) e = w;
+        }
         if (e != hipSuccess) return e;
     }
     bool ok = true;

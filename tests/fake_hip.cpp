@@ -21,6 +21,8 @@ struct Launch { std::string kernel; uint32_t grid, block; size_t lds; int stream
 
 std::recursive_mutex mu;
 int queues = 4, streams_made = 0, streams_alive = 0, streams_limit = 1 << 30, busy = 0;
+int launches_left = 1 << 30, last_error = 0;
+std::map<void*, int> unfinished;   // launches of a stream that nothing has waited for
 size_t host_limit = SIZE_MAX;
 std::vector<size_t> allocations;   // of device memory, in bytes
 std::vector<int> users;
@@ -49,6 +51,12 @@ void fake_streams_limit(int n) { streams_limit = n; }
 void fake_busy(int on) { busy = on; }
 void fake_host_limit(size_t bytes) { host_limit = bytes; }
 int fake_streams_alive() { return streams_alive; }
+void fake_launches_left(int n) { launches_left = n; }
+int fake_unfinished() {
+    int n = 0;
+    for (const auto& s : unfinished) n += s.second;
+    return n;
+}
 void fake_clear() { launches.clear(); allocations.clear(); }
 int fake_allocations_of(size_t bytes) {
     int n = 0;
@@ -82,7 +90,9 @@ int hipLaunchKernel(const void* f, dim3_ g, dim3_ b, void** args, size_t lds, vo
     Stream* st = (Stream*)s;
     const int q = st ? st->queue : 0;
     const std::string& name = names[f];
+    if (launches_left-- <= 0) return last_error = 719;   // a launch failure
     launches.push_back({name, g.x, b.x, lds, st ? st->id : -1, q});
+    unfinished[s]++;
     if (name.find("k_hold") != std::string::npos) {   // (uint64_t* span, uint32_t ticks of 10 ns)
         uint64_t* span = *(uint64_t**)args[0];
         const uint64_t ticks = *(uint32_t*)args[1];
@@ -115,11 +125,13 @@ int hipStreamDestroy(void* s) {
     std::lock_guard<std::recursive_mutex> l(mu);
     users[((Stream*)s)->queue]--;
     streams_alive--;
+    unfinished.erase(s);
     delete (Stream*)s;
     return 0;
 }
-int hipStreamSynchronize(void*) {
+int hipStreamSynchronize(void* s) {
     std::lock_guard<std::recursive_mutex> l(mu);
+    unfinished.erase(s);
     for (uint64_t t : queue_free) now = t > now ? t : now;
     return 0;
 }
@@ -173,7 +185,11 @@ int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int thread
     *n = 1024 / threads;   // 16 wavefronts
     return 0;
 }
-int hipGetLastError() { return 0; }
+int hipGetLastError() {
+    const int e = last_error;
+    last_error = 0;
+    return e;
+}
 const char* hipGetErrorString(int) { return "fake error"; }
 
 }  // extern "C"

@@ -130,6 +130,21 @@ print(json.dumps([got, fake.fake_streams_alive()]))
     assert len(got) == 2 and alive == 0
 
 
+@pytest.mark.parametrize("launches", [1, 2, 3, 4, 6, 9])
+def test_a_failed_launch_in_the_search_leaves_nothing_running(fake, launches):
+    """The search's kernels write to the memory that pose calls use: none may be
+    left in flight, whichever launch fails, and the job is not refused."""
+    left, groups = run(fake, """
+ctx = context()
+fake.fake_launches_left(%d)
+j = job(ctx, ls="none")
+left = fake.fake_unfinished()
+fake.fake_launches_left(1 << 30)
+print(json.dumps([left, len(launched(lambda: j.run(1), "k_gen"))]))
+""" % launches, 8)
+    assert left == 0 and groups == 4
+
+
 def test_searches_for_lanes_become_rare(fake):
     """Where there are no lanes to be found, 32 jobs look for them 6 times."""
     got = run(fake, """
