@@ -1275,13 +1275,15 @@ inline Shape choose_shape(const LigandDev& L, int team_width_hint, bool grad, in
 // FIRE, nrun 60 185 against 147, Solis-Wets 165 against 127.  A server's
 // launches keep 256 threads: larger workgroups need half or all of a compute
 // unit free at once, which the launches of other requests seldom leave (24
-// ligands in 16 slots 0.56 s against 0.50 s).  So do ADADELTA's (uneven) where
-// others would take more than 512 or read PairC: a workgroup keeps its place
-// until its last search ends, and ADADELTA's differ in length by ten times.  M
-// evals/s in 256 threads against that: 60 atoms, nrun 50 / 100 147 / 202
-// against 132 / 182; 72 atoms, nrun 50 145 against 131; 90 atoms, nrun 40 / 100
-// 49 / 91 against 42 / 73.  (In 512 threads 54 atoms ran 221 against 230 at
-// nrun 50, 288 against 269 at nrun 100 and, on 126^3 maps, 283 against 260.)
+// ligands in 16 slots 0.56 s against 0.50 s).  So do ADADELTA's (uneven) of
+// more searches than fit at once, unless 512 hold records that 256 leave in
+// memory: a workgroup keeps its place until its last search ends, and
+// ADADELTA's differ in length by ten times.  M evals/s in 256 threads against
+// what other searches take there: 45 atoms, nrun 50 293 against 242 (on 126^3
+// maps 330 against 367); 60 atoms, nrun 50 / 100 147 / 202 against 132 / 182;
+// 72 atoms, nrun 50 86 against 73; 90 atoms, nrun 40 / 100 49 / 91 against 42 /
+// 73.  54 atoms, in 512: nrun 50 / 100 221 / 288 against 230 / 269, on 126^3
+// maps 283 / 311 against 260 / 278.
 // fixed: the threads if they are not to be chosen, else 0.
 inline Shape choose_ls_shape(const LaunchArgs& la, int searches, bool grad, int fixed, bool uneven = false) {
     const LigandDev& L = *la.lig_host;
@@ -1289,13 +1291,14 @@ inline Shape choose_ls_shape(const LaunchArgs& la, int searches, bool grad, int 
     if (la.crowded || fixed) return s;
     // wavefronts of all the launches that share the device, were they like this one
     const int64_t need = ((int64_t)searches * s.tw + kWave - 1) / kWave * la.share;
+    const bool small = s.pl || compact_pairs(s.tw * s.nc, grad);   // uneven searches stay in 256 threads
     int64_t best = INT64_MIN;
     for (int t = kGroupThreads; t <= 4 * kGroupThreads; t += kGroupThreads) {   // whole rounds of the four SIMDs
         const size_t lds = lds_bytes_for(s.tw, s.nc, L.num_rotbonds, L.num_pairs, true, grad, t);
         const int w = t / kWave, fit = groups_per_cu(lds, t);
         const int64_t groups = (need + w - 1) / w;
         const bool all = groups <= (int64_t)fit * kCus;
-        if (!all && (fit * w < 12 || (uneven && (t > 2 * kGroupThreads || compact_pairs(s.tw * s.nc, grad))))) continue;
+        if (!all && (fit * w < 12 || (uneven && (small || t > 2 * kGroupThreads)))) continue;
         // all at once: prefer few wavefronts on the fullest compute unit; else many in all
         const int64_t score = all ? 2 * kCuWaves - (groups + kCus - 1) / kCus * w : fit * w - kCuWaves;
         if (score > best) {

@@ -206,7 +206,7 @@ print(json.dumps([threads(72, 10, 64, 40, ls) for ls in ("sw", "ad", "adam", "fi
 # threads of the workgroups that a launch of all their searches takes
 LARGE = [(54, 8, 32, "adam", 80, 512), (66, 10, 32, "sw", 80, 512), (80, 12, 32, "adam", 20, 512),
          (80, 12, 32, "fire", 40, 768), (66, 10, 32, "adam", 80, 1024), (80, 12, 32, "sw", 80, 1024),
-         (60, 10, 64, "sw", 40, 512), (54, 8, 64, "ad", 80, 512), (64, 10, 64, "ad", 20, 768), (84, 12, 64, "sw", 20, 768),
+         (60, 10, 64, "sw", 40, 512), (56, 14, 64, "ad", 80, 512), (64, 10, 64, "ad", 20, 768), (84, 12, 64, "sw", 20, 768),
          (64, 10, 64, "adam", 40, 1024), (84, 12, 64, "fire", 40, 1024), (84, 12, 64, "sw", 40, 1024)]
 
 
@@ -220,10 +220,10 @@ print(json.dumps([[threads(*c[:3], n, c[3]) for n in (c[4], 2)] for c in %r]))
     assert got == [[c[5], 256] for c in LARGE]
 
 
-@pytest.mark.parametrize("atoms, width", [(64, 64), (66, 64), (84, 64), (80, 32)])
+@pytest.mark.parametrize("atoms, width", [(48, 64), (64, 64), (66, 64), (84, 64), (80, 32)])
 def test_many_uneven_searches_stay_in_small_workgroups(fake, atoms, width):
     """ADADELTA launches that do not hold all their searches at once, where
-    ADAM's take 512 to 1024 threads."""
+    ADAM's take 512 to 1024 threads (56 atoms take 512: LARGE)."""
     ad, adam = run(fake, WORKGROUPS + """
 print(json.dumps([threads(%d, 10, %d, 80, ls) for ls in ("ad", "adam")]))
 """ % (atoms, width))
